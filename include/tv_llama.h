@@ -36,8 +36,9 @@ extern "C" {
 #define TV_EPI_LOGITS 2  /* out: float [M, N] (may be NULL) + per-work-group argmax keys */
 
 /*
- * K elements per split that tv_llama_decode_step uses for an M x N x K product
- * (a multiple of 32; >= K means one split).  Host-only.
+ * K elements per split that tv_llama_decode_step and tv_llama_prefill use for an
+ * M x N x K product of a 16-bit model (a multiple of 32; >= K means one split).
+ * Host-only.
  */
 int tv_linear_k_split(int M, int N, int K);
 

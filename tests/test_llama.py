@@ -126,6 +126,53 @@ def test_linear_logits_and_greedy(M, N, K, dtype):
     assert np.array_equal(toks.cpu().numpy(), np.argmax(logits.cpu().numpy(), axis=1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (128, 128, 64, 64), (129, 132, 96, 96),      # 64 x 128 tiles
+                                      (191, 260, 1056, 352), (320, 256, 2048, 512),
+                                      (129, 16400, 160, 160),
+                                      (200, 32000, 128, 64), (257, 32772, 32, 32),                  # 128 x 128
+                                      (300, 32000, 96, 96), (513, 16392, 160, 160)])                # 256 x 256
+def test_linear_many_rows(dtype, M, N, K, ks):
+    """More than 64 rows: each tile shape at its edges (rows, features and K past the last
+    tile, short last stages, splits that are not whole stages), A rows at a stride, the
+    three epilogues on the same products.  fp32 sums of exact products: the error of a sum
+    of K terms is below K * 2^-24 of the sum of magnitudes, at most 2e-5 of it here."""
+    from tinyvllm_amd._lib import dtype_code
+    lda = K + 8
+    a = gen(40, M, lda, dtype=dtype)[:, :K]
+    w = gen(41, N, K, dtype=dtype, scale=0.05)
+    code = dtype_code(dtype)
+    splits = -(-K // ks)
+    part = torch.full((splits, M, N), float("nan"), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(part), ptr(a), ptr(w), M, N, K, lda, 0, ks, 0, None, code, None), "partial")
+    logits = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    keys = torch.zeros((-(-N // 64), M), dtype=torch.int64, device="cuda")
+    check(lib().tv_linear(ptr(logits), ptr(a), ptr(w), M, N, K, lda, N, K, 2, ptr(keys), code, None), "logits")
+    toks = torch.zeros(M, dtype=torch.int32, device="cuda")
+    check(lib().tv_argmax_advance(ptr(toks), None, None, None, 0, ptr(keys), keys.shape[0], M, None), "argmax")
+    # SwiGLU rows at a 16-byte pitch (one store per lane) and at one that is only 4-byte aligned
+    outs = [torch.full((M, ldo), float("nan"), dtype=dtype, device="cuda") for ldo in (-(-N // 16) * 8, N // 2 + 2)]
+    for o in outs:
+        check(lib().tv_linear(ptr(o), ptr(a), ptr(w), M, N, K, lda, o.shape[1], K, 1, None, code, None), "swiglu")
+    torch.cuda.synchronize()
+    A, W = f64(a), f64(w)
+    mag = np.abs(A) @ np.abs(W).T
+    P = part.double().cpu().numpy()
+    for s in range(splits):
+        k = slice(s * ks, (s + 1) * ks)
+        assert (np.abs(P[s] - A[:, k] @ W[:, k].T) <= 2e-5 * mag).all(), s
+    want = A @ W.T
+    assert (np.abs(f64(logits) - want) <= 2e-5 * mag).all()
+    assert np.array_equal(toks.cpu().numpy(), np.argmax(logits.cpu().numpy(), axis=1))
+    y = want.reshape(M, N // 4, 2, 2)
+    g, u = y[:, :, 0].reshape(M, -1), y[:, :, 1].reshape(M, -1)
+    sw = g / (1 + np.exp(-g)) * u
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8       # one rounding to the output type
+    for o in outs:
+        assert (np.abs(f64(o[:, :N // 2]) - sw) <= 1.01 * eps * np.abs(sw) + 1e-4).all()
+        assert torch.isnan(o[:, N // 2:]).all()                        # nothing past the row
+
+
 def test_greedy_tie_resolves_to_first_index():
     """Two identical, dominant rows in different work-group tiles (5 and 70): every
     token ties between them and must take 5 (numpy / tinygrad argmax semantics)."""

@@ -36,6 +36,26 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 int splits_of(int K, int k_split) { return (K + k_split - 1) / k_split; }
 
+// Work-groups a skinny product aims for when it splits K.
+constexpr long long kLinearTargetWorkGroups = 192;
+
+// K elements per split of a product whose consumer sums the partials.
+int k_split_of(int M, int N, int K, int dtype) {
+  if (M > tv::kLinBM && dtype != TV_F32) return tv::tile_linear_k_split(M, N, K);
+  const long long full = round_up(K, 32);
+  const long long tiles = ((N + tv::kLinBN - 1) / tv::kLinBN) * (long long)((M + tv::kLinBM - 1) / tv::kLinBM);
+  // About three work-groups per four CUs: more splits add partials that the
+  // consumer (norm or step attention) reads back, and on the TinyLlama step
+  // 192 beat 128, 160, 224 and 256 (1.53 vs 1.55-1.59 ms).
+  const long long target = kLinearTargetWorkGroups;
+  if (tiles >= target / 2) return (int)full;
+  const long long want = (target + tiles - 1) / tiles;
+  const long long per = (K + want - 1) / want;
+  // whole LDS chunks: a partial chunk still streams the chunk's full width of W
+  const long long ks = per >= tv::kLinKC ? (per + tv::kLinKC / 2) / tv::kLinKC * tv::kLinKC : round_up(per, 32);
+  return (int)std::min(full, std::max(ks, 32LL));
+}
+
 // Carves 256-byte aligned regions out of one workspace.
 struct Carver {
   size_t off = 0;
@@ -79,9 +99,9 @@ StepLayout step_layout(const tv_llama_model* m, int B, int max_blocks, int block
   const int qd = m->n_heads * m->head_dim;
   const int kd = m->n_kv_heads * m->head_dim;
   const int nqkv = qkv_width(m);
-  L.ks_qkv = tv_linear_k_split(B, nqkv, m->dim);
-  L.ks_o = tv_linear_k_split(B, m->dim, qd);
-  L.ks_2 = tv_linear_k_split(B, m->dim, m->hidden_dim);
+  L.ks_qkv = k_split_of(B, nqkv, m->dim, m->dtype);
+  L.ks_o = k_split_of(B, m->dim, qd, m->dtype);
+  L.ks_2 = k_split_of(B, m->dim, m->hidden_dim, m->dtype);
   const size_t part_floats = std::max({(size_t)splits_of(m->dim, L.ks_qkv) * nqkv, (size_t)splits_of(qd, L.ks_o) * m->dim,
                                        (size_t)splits_of(m->hidden_dim, L.ks_2) * m->dim}) * (size_t)B;
   const size_t es = elem_bytes(m->dtype);
@@ -313,27 +333,13 @@ int run_layers(const tv_llama_model* m, const tv_llama_cache* c, const LayerIO& 
   return TV_OK;
 }
 
-// Work-groups a skinny product aims for when it splits K.
-constexpr long long kLinearTargetWorkGroups = 192;
-
 }  // namespace
 
 extern "C" {
 
 int tv_linear_k_split(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 32;
-  const long long full = round_up(K, 32);
-  const long long tiles = ((N + tv::kLinBN - 1) / tv::kLinBN) * (long long)((M + tv::kLinBM - 1) / tv::kLinBM);
-  // About three work-groups per four CUs: more splits add partials that the
-  // consumer (norm or step attention) reads back, and on the TinyLlama step
-  // 192 beat 128, 160, 224 and 256 (1.53 vs 1.55-1.59 ms).
-  const long long target = kLinearTargetWorkGroups;
-  if (tiles >= target / 2) return (int)full;
-  const long long want = (target + tiles - 1) / tiles;
-  const long long per = (K + want - 1) / want;
-  // whole LDS chunks: a partial chunk still streams the chunk's full width of W
-  const long long ks = per >= tv::kLinKC ? (per + tv::kLinKC / 2) / tv::kLinKC * tv::kLinKC : round_up(per, 32);
-  return (int)std::min(full, std::max(ks, 32LL));
+  return k_split_of(M, N, K, TV_F16);
 }
 
 int tv_linear(void* out, const void* a, const void* w, int M, int N, int K, int64_t lda, int64_t ldo, int k_split,

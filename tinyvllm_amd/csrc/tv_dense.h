@@ -96,6 +96,10 @@ bool step_attn_supported(int head_dim, int group, int block_size);
 void launch_step_attn(const StepAttnParams& p, int head_dim, int dtype, hipStream_t s);
 
 void launch_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
+// many-row products (tile_linear.hip)
+bool tile_linear_supported(const LinearParams& p, int dtype);
+int tile_linear_k_split(int M, int N, int K);
+void launch_tile_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
 void launch_norm(const NormParams& p, int dtype, hipStream_t s);
 void launch_qkv_rope(const QKVParams& p, int dtype, hipStream_t s);
 void launch_rope_table(float* table, int max_pos, int head_dim, float theta, hipStream_t s);
