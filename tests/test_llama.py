@@ -126,17 +126,8 @@ def test_linear_logits_and_greedy(M, N, K, dtype):
     assert np.array_equal(toks.cpu().numpy(), np.argmax(logits.cpu().numpy(), axis=1))
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (128, 128, 64, 64), (129, 132, 96, 96),      # 64 x 128 tiles
-                                      (191, 260, 1056, 352), (320, 256, 2048, 512),
-                                      (129, 16400, 160, 160),
-                                      (200, 32000, 128, 64), (257, 32772, 32, 32),                  # 128 x 128
-                                      (300, 32000, 96, 96), (513, 16392, 160, 160)])                # 256 x 256
-def test_linear_many_rows(dtype, M, N, K, ks):
-    """More than 64 rows: each tile shape at its edges (rows, features and K past the last
-    tile, short last stages, splits that are not whole stages), A rows at a stride, the
-    three epilogues on the same products.  fp32 sums of exact products: the error of a sum
-    of K terms is below K * 2^-24 of the sum of magnitudes, at most 2e-5 of it here."""
+def check_products(dtype, M, N, K, ks):
+    """The three epilogues of one product against 64 bits, A rows at a stride."""
     from tinyvllm_amd._lib import dtype_code
     lda = K + 8
     a = gen(40, M, lda, dtype=dtype)[:, :K]
@@ -167,10 +158,34 @@ def test_linear_many_rows(dtype, M, N, K, ks):
     y = want.reshape(M, N // 4, 2, 2)
     g, u = y[:, :, 0].reshape(M, -1), y[:, :, 1].reshape(M, -1)
     sw = g / (1 + np.exp(-g)) * u
-    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8       # one rounding to the output type
+    eps = torch.finfo(dtype).eps / 2       # one rounding to the output type
     for o in outs:
         assert (np.abs(f64(o[:, :N // 2]) - sw) <= 1.01 * eps * np.abs(sw) + 1e-4).all()
         assert torch.isnan(o[:, N // 2:]).all()                        # nothing past the row
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (128, 128, 64, 64), (129, 132, 96, 96),      # 64 x 128 tiles
+                                      (191, 260, 1056, 352), (320, 256, 2048, 512),
+                                      (129, 16400, 160, 160),
+                                      (200, 32000, 128, 64), (257, 32772, 32, 32),                  # 128 x 128
+                                      (300, 32000, 96, 96), (513, 16392, 160, 160)])                # 256 x 256
+def test_linear_many_rows(dtype, M, N, K, ks):
+    """More than 64 rows: each tile shape at its edges (rows, features and K past the last
+    tile, short last stages, splits that are not whole stages), A rows at a stride, the
+    three epilogues on the same products.  fp32 sums of exact products: the error of a sum
+    of K terms is below K * 2^-24 of the sum of magnitudes, at most 2e-5 of it here."""
+    check_products(dtype, M, N, K, ks)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N,K,ks", [(1, 4, 32, 32),                      # one row, one short stage
+                                      (4, 1028, 1056, 352),                # splits that are not whole stages
+                                      (3, 8196, 96, 96), (5, 4100, 544, 256),  # several units per work-group
+                                      (16, 2064, 2080, 1024), (8, 16452, 160, 160)])
+def test_linear_few_rows(dtype, M, N, K, ks):
+    """At most 16 rows: waves without a stage, rings that run across units, ragged N and K."""
+    check_products(dtype, M, N, K, ks)
 
 
 def test_greedy_tie_resolves_to_first_index():

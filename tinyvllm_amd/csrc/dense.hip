@@ -8,7 +8,8 @@
 //   greedy sampling  argmax over the vocabulary (first maximum)  sampling.py:131-134
 //
 // linear_kernel computes Y = A W^T for a skinny A (the decode batch, M <= 64
-// per work-group; products of more rows at 16 bits: tile_linear.hip) against a weight matrix W [N, K] that is streamed from HBM
+// per work-group; at most 16 rows: few_linear_kernel; more than 64 at 16 bits:
+// tile_linear.hip) against a weight matrix W [N, K] that is streamed from HBM
 // exactly once.  Each of the 4 waves of a work-group owns 16 rows of W and all
 // 64 rows of A; A is staged in LDS per 512-byte-wide K chunk (256 fp16/bf16 or
 // 128 fp32 elements) and shared by the waves.  fp32 runs the same byte layout
@@ -18,6 +19,9 @@
 #include "tv_common.h"
 #include "tv_dense.h"
 #include "tv_linear.h"
+#include "tv_tile_dma.h"
+
+#include <algorithm>
 
 namespace tv {
 
@@ -39,19 +43,20 @@ constexpr int lcm3(int a, int b, int c) {
   return ab / gcd_c(ab, c) * c;
 }
 
-// Epilogue of the skinny product: lane (wave, g, col) holds acc[mb][i] =
-// Y[m0 + 16 mb + col][n_wave + 4 g + i].  sk: 8 KB of LDS for the argmax
-// exchange (logits), free to reuse once every wave reaches this point.
-template <typename T, int EPI>
-__device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32x4 (&acc)[4], int n_wave, int m0,
+// Epilogue of the skinny products: lane (wave, g, col) holds acc[mb][i] =
+// Y[m0 + 16 mb + col][n_wave + 4 g + i].  sk: 2 KB of LDS per 16 rows for the
+// argmax exchange (logits), free to reuse once every wave reaches this point.
+template <typename T, int EPI, int MB>
+__device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32x4 (&acc)[MB], int n_wave, int m0,
                                                 int split, int ntile, int wave, int tid, unsigned long long* sk) {
+  constexpr int ROWS = 16 * MB;
   const int lane = tid & 63;
   const int g = lane >> 4;
   const int col = lane & 15;
   const int n = n_wave + 4 * g;
   if constexpr (EPI == kEpiPartial) {
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
+    for (int mb = 0; mb < MB; ++mb) {
       const int m = m0 + mb * 16 + col;
       if (m < p.M && n < p.N)
         *reinterpret_cast<f32x4*>(p.part + ((size_t)split * p.M + m) * p.N + n) = acc[mb];
@@ -59,7 +64,7 @@ __device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32
   } else if constexpr (EPI == kEpiSwiglu) {
     // rows 4j, 4j+1 of W are w1 rows 2j, 2j+1; rows 4j+2, 4j+3 the matching w3 rows
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
+    for (int mb = 0; mb < MB; ++mb) {
       const int m = m0 + mb * 16 + col;
       if (m < p.M && n < p.N) {
         const f32x4 v = acc[mb];
@@ -67,9 +72,9 @@ __device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32
       }
     }
   } else {
-    lds_barrier();   // sk reuses LDS of the main loop: [16 (wave, g)][64 rows]
+    lds_barrier();   // sk reuses LDS of the main loop: [16 (wave, g)][ROWS]
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
+    for (int mb = 0; mb < MB; ++mb) {
       const int m = m0 + mb * 16 + col;
       const f32x4 v = acc[mb];
       if (p.out && m < p.M && n < p.N)
@@ -78,13 +83,13 @@ __device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (n + i < p.N) best = max(best, argmax_key(v[i], n + i));
-      sk[(wave * 4 + g) * 64 + mb * 16 + col] = best;
+      sk[(wave * 4 + g) * ROWS + mb * 16 + col] = best;
     }
     lds_barrier();
-    if (tid < 64 && p.keys && m0 + tid < p.M) {
+    if (tid < ROWS && p.keys && m0 + tid < p.M) {
       unsigned long long best = sk[tid];
 #pragma unroll
-      for (int j = 1; j < 16; ++j) best = max(best, sk[j * 64 + tid]);
+      for (int j = 1; j < 16; ++j) best = max(best, sk[j * ROWS + tid]);
       p.keys[(size_t)ntile * p.M + m0 + tid] = best;
     }
   }
@@ -232,29 +237,176 @@ __global__ void __launch_bounds__(256, kLinearMinBlocks) linear_kernel(const Lin
     }
   }
 
-  linear_epilogue<T, EPI>(p, acc, n_wave, m0, split, ntile, wave, tid, reinterpret_cast<unsigned long long*>(&sa[0][0]));
+  linear_epilogue<T, EPI, 4>(p, acc, n_wave, m0, split, ntile, wave, tid, reinterpret_cast<unsigned long long*>(&sa[0][0]));
 }
 
 
-#define TV_LINEAR_CASE(T)                                                                              \
-  switch (epi) {                                                                                       \
-    case kEpiPartial: hipLaunchKernelGGL((linear_kernel<T, kEpiPartial>), grid, dim3(256), 0, s, p); \
-      break;                                                                                           \
-    case kEpiSwiglu: hipLaunchKernelGGL((linear_kernel<T, kEpiSwiglu>), grid, dim3(256), 0, s, p);   \
-      break;                                                                                           \
-    default: hipLaunchKernelGGL((linear_kernel<T, kEpiLogits>), grid, dim3(256), 0, s, p);           \
+// The product for at most kFewRows rows of A, where the time should be the
+// stream of W.  Every wave has a ring of S stages in LDS, each 512 bytes of 16
+// rows of W and of RA rows of A, filled by direct loads (512 contiguous bytes
+// per row and instruction).  The ring is private to the wave, so no barrier
+// stands between its loads.  KW = 4: a unit is 16 rows of W, whose stages the
+// waves take in turn and sum through LDS, so even a product of 2048 features
+// has a unit for every CU with few splits.  KW = 1: 64 rows, 16 per wave (the
+// logits, whose argmax keys cover 64 features).  One work-group per CU walks
+// the units; its loads run ahead across them.  The 64-row kernel spent its
+// time on products for rows that are not there (fp32) and on one 64-row tile
+// per work-group, 176 of them on 256 CUs.  MI355X, 4 rows, against it:
+// 11264 x 2048 fp32 47 -> 20.0 us (4.6 TB/s), 32000 x 2048 87 -> 47.7 (5.5),
+// 2048 x 5632 26 -> 12.5; fp16 15.9 -> 11.3, 31.4 -> 24.9, 9.4 -> 7.3.  At 16
+// rows, fp16: 16.4 -> 13.5, 31.7 -> 26.3, 9.9 -> 8.6.  Rejected: A held in LDS
+// with W in registers (fp32 25.9 / 62.9 / 12.6 us), both in registers (29.1 /
+// 56.0 / 13.8); there an instruction reads 64 bytes of 16 rows.
+template <typename T, int EPI, int KW, int RA, int S>
+__global__ void __launch_bounds__(256) few_linear_kernel(const LinearParams p) {
+  constexpr int ES = (int)sizeof(T);
+  constexpr int CB = kFewStage;
+  constexpr int LW = 8, LA = RA / 2;   // loads per stage: two rows each
+  constexpr int STAGE = (16 + RA) * CB;
+  __shared__ __attribute__((aligned(1024))) uint8_t sm[4 * S * STAGE];
+  __shared__ f32x4 red[2][256];        // sums of the waves (KW = 4), argmax keys (logits)
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int g = lane >> 4;
+  const int col = lane & 15;
+  const int kw = KW == 4 ? wave : 0;
+  const int ntiles = (p.N + 64 / KW - 1) / (64 / KW);
+  const int splits = (p.K + p.k_split - 1) / p.k_split;
+  const int units = ntiles * splits;   // consecutive units: the splits of one n tile
+
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)sm + wave * S * STAGE;
+  const uint8_t* const ring = sm + wave * S * STAGE;
+  auto stages_of = [&](int split) {    // of this wave: kw, kw + KW, ...
+    const int nc = (min(p.k_split, p.K - split * p.k_split) * ES + CB - 1) / CB;
+    return (nc - kw + KW - 1) / KW;
+  };
+
+  // the unit that is being loaded
+  struct Source {
+    u32x4 wres, ares;
+    int kbytes, nc, ni, rot, rows_w, i;
+  } src;
+  int lu = blockIdx.x;
+  auto open = [&]() {
+    const int ntile = lu / splits, split = lu - ntile * splits;
+    const int kb = split * p.k_split;
+    const int n_wave = KW == 4 ? ntile * 16 : ntile * 64 + wave * 16;
+    src.kbytes = min(p.k_split, p.K - kb) * ES;
+    src.nc = (src.kbytes + CB - 1) / CB;
+    src.ni = stages_of(split);
+    // n tiles start at scattered columns: with rows of W a power of two apart,
+    // work-groups in step at one column keep to a few HBM channels (4096 x
+    // 16384 fp32: 68.9 us from 16 starting columns, 49.3 from all; 53.7 at a
+    // row of 17408, where the start does not matter)
+    src.rot = (int)(((((uint32_t)ntile * 0x9E3779B1u) >> 16) * (uint32_t)src.nc) >> 16);
+    // ranges end at the wave's last row; everything else (rows past N or M, K
+    // past the split, stages past the last) is sent out of range by bit 31 and
+    // reads zero
+    src.rows_w = min(16, max(p.N - n_wave, 0));
+    src.wres = rsrc_words(reinterpret_cast<const T*>(p.w) + (size_t)min(n_wave, p.N) * p.K + kb,
+                          src.rows_w ? ((unsigned long long)src.rows_w * p.K - kb) * ES : 0);
+    src.ares = rsrc_words(reinterpret_cast<const T*>(p.a) + kb,
+                          ((unsigned long long)(p.M - 1) * p.lda + p.K - kb) * ES);
+    src.i = 0;
+  };
+  // Load i of a stage covers rows 2 i and 2 i + 1: lane -> row lane / 32, slot
+  // lane % 32; 16-byte chunk c of row r sits at slot c ^ r, so the 16 rows of
+  // a fragment read fall on distinct banks.
+  const int lrow = lane >> 5;
+  auto load = [&](uint32_t base) {
+    while (lu < units && src.i >= src.ni) {
+      lu += gridDim.x;
+      if (lu < units) open();
+    }
+    int c = kw + KW * src.i + src.rot;
+    c = c < src.nc ? c : c - src.nc;
+    const int left = lu < units ? src.kbytes - c * CB : 0;   // bytes of this stage
+    ++src.i;
+#pragma unroll
+    for (int t = 0; t < LW; ++t) {
+      const int r = 2 * t + lrow, o = 16 * ((lane & 31) ^ r);
+      const bool in = o < left && r < src.rows_w;
+      load_lds16(src.wres, base + t * 1024, in ? (uint32_t)(r * p.K * ES + c * CB + o) : 0x80000000u);
+    }
+#pragma unroll
+    for (int t = 0; t < LA; ++t) {
+      const int r = 2 * t + lrow, o = 16 * ((lane & 31) ^ r);
+      const bool in = o < left && r < p.M;
+      load_lds16(src.ares, base + (LW + t) * 1024, in ? (uint32_t)(r * (int)p.lda * ES + c * CB + o) : 0x80000000u);
+    }
+  };
+
+  const int ar = col & (RA - 1);       // columns past RA read copies; columns past M are dropped
+  open();
+#pragma unroll
+  for (int j = 0; j < S; ++j) load(ring0 + j * STAGE);
+  int at = 0, parity = 0;
+  for (int u = blockIdx.x; u < units; u += gridDim.x) {
+    const int ntile = u / splits, split = u - ntile * splits;
+    const int ni = stages_of(split);
+    f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+    for (int i = 0; i < ni; ++i) {
+      wait_vmcnt<(S - 1) * (LW + LA)>();
+      const uint8_t* st = ring + at;
+      u32x4 w[8], a[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        w[s] = *reinterpret_cast<const u32x4*>(st + col * CB + 16 * ((4 * s + g) ^ col));
+        a[s] = *reinterpret_cast<const u32x4*>(st + (16 + ar) * CB + 16 * ((4 * s + g) ^ ar));
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the stage is in registers, its buffer free
+      load(ring0 + at);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) acc[0] = mfma_frag<T>(w[s], a[s], acc[0]);
+      at = at == (S - 1) * STAGE ? 0 : at + STAGE;
+    }
+    if constexpr (KW == 4) {
+      // two buffers: a wave passes the next unit's barrier only after wave 0 has read this one's
+      red[parity][tid] = acc[0];
+      lds_barrier();
+      if (wave == 0) {
+        acc[0] = (red[parity][lane] + red[parity][64 + lane]) + (red[parity][128 + lane] + red[parity][192 + lane]);
+        linear_epilogue<T, EPI, 1>(p, acc, ntile * 16, 0, split, ntile, wave, tid, nullptr);
+      }
+      parity ^= 1;
+    } else {
+      linear_epilogue<T, EPI, 1>(p, acc, ntile * 64 + wave * 16, 0, split, ntile, wave, tid,
+                                 reinterpret_cast<unsigned long long*>(&red[0][0]));
+    }
   }
+  wait_vmcnt<0>();                     // loads still under way write zeros to the ring
+}
+
+template <typename T, int EPI> static void launch_few(const LinearParams& p, hipStream_t s) {
+  constexpr int KW = EPI == kEpiLogits ? 1 : 4;
+  const long long units = (long long)((p.N + 64 / KW - 1) / (64 / KW)) * ((p.K + p.k_split - 1) / p.k_split);
+  const dim3 grid((unsigned)std::min<long long>(units, kFewWorkGroups));
+  if (p.M <= 4) hipLaunchKernelGGL((few_linear_kernel<T, EPI, KW, 4, 3>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((few_linear_kernel<T, EPI, KW, 16, 2>), grid, dim3(256), 0, s, p);
+}
+
+template <typename T> static void launch_linear_t(const LinearParams& p, int epi, hipStream_t s) {
+  constexpr long long ES = sizeof(T);
+  if (p.M <= kFewRows && std::max<long long>(p.lda, p.K) * ES * 16 < (1LL << 31)) {   // 32-bit offsets in 16 rows
+    if (epi == kEpiPartial) launch_few<T, kEpiPartial>(p, s);
+    else if (epi == kEpiSwiglu) launch_few<T, kEpiSwiglu>(p, s);
+    else launch_few<T, kEpiLogits>(p, s);
+    return;
+  }
+  const dim3 grid((p.K + p.k_split - 1) / p.k_split, (p.N + kLinBN - 1) / kLinBN, (p.M + kLinBM - 1) / kLinBM);
+  if (epi == kEpiPartial) hipLaunchKernelGGL((linear_kernel<T, kEpiPartial>), grid, dim3(256), 0, s, p);
+  else if (epi == kEpiSwiglu) hipLaunchKernelGGL((linear_kernel<T, kEpiSwiglu>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((linear_kernel<T, kEpiLogits>), grid, dim3(256), 0, s, p);
+}
 
 void launch_linear(const LinearParams& p, int epi, int dtype, hipStream_t s) {
   if (tile_linear_supported(p, dtype)) return launch_tile_linear(p, epi, dtype, s);
-  const dim3 grid((p.K + p.k_split - 1) / p.k_split, (p.N + kLinBN - 1) / kLinBN, (p.M + kLinBM - 1) / kLinBM);
-  if (dtype == kF16) {
-    TV_LINEAR_CASE(_Float16)
-  } else if (dtype == kBF16) {
-    TV_LINEAR_CASE(__bf16)
-  } else {
-    TV_LINEAR_CASE(float)
-  }
+  if (dtype == kF16) launch_linear_t<_Float16>(p, epi, s);
+  else if (dtype == kBF16) launch_linear_t<__bf16>(p, epi, s);
+  else launch_linear_t<float>(p, epi, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -39,9 +39,34 @@ int splits_of(int K, int k_split) { return (K + k_split - 1) / k_split; }
 // Work-groups a skinny product aims for when it splits K.
 constexpr long long kLinearTargetWorkGroups = 192;
 
+// K elements per split of a product of at most kFewRows rows (few_linear_kernel):
+// the cheapest of 1 .. 8 splits, in the stages that the busiest work-group
+// walks (its units, each the stages of one wave times four and about three more
+// to start and sum; two more per split for the partials).  MI355X, 4 rows,
+// 1 / 2 / 3 / 4 splits: 2048 x 5632 fp32 14.4 / 12.5 / 13.4 / 12.1 us (takes 2),
+// fp16 8.8 / 7.3 / 7.9 / 7.6 (2); 2560 x 2048 fp16 5.1 / 5.4 / 5.6 / 5.7 (1);
+// 1024 x 2816 fp32 9.0 / 6.7 / 6.1 / 5.9 (3).
+int few_k_split(int N, int K, int es) {
+  const int nc = (K * es + tv::kFewStage - 1) / tv::kFewStage;
+  const long long tiles = (N + 15) / 16;
+  long long best = 0;
+  int chunks = nc;
+  for (int s = 1; s <= 8 && s <= nc; ++s) {
+    const int per = (nc + s - 1) / s;
+    const long long rounds = (tiles * s + tv::kFewWorkGroups - 1) / tv::kFewWorkGroups;
+    const long long cost = rounds * ((per + 3) / 4 * 4 + 3) + 2 * (s - 1);
+    if (s == 1 || cost < best) {
+      best = cost;
+      chunks = per;
+    }
+  }
+  return (int)std::min<long long>(round_up(K, 32), (long long)chunks * (tv::kFewStage / es));
+}
+
 // K elements per split of a product whose consumer sums the partials.
 int k_split_of(int M, int N, int K, int dtype) {
   if (M > tv::kLinBM && dtype != TV_F32) return tv::tile_linear_k_split(M, N, K);
+  if (M <= tv::kFewRows) return few_k_split(N, K, (int)elem_bytes(dtype));
   const long long full = round_up(K, 32);
   const long long tiles = ((N + tv::kLinBN - 1) / tv::kLinBN) * (long long)((M + tv::kLinBM - 1) / tv::kLinBM);
   // About three work-groups per four CUs: more splits add partials that the

@@ -10,6 +10,9 @@ enum LinearEpilogue : int { kEpiPartial = 0, kEpiSwiglu = 1, kEpiLogits = 2 };
 
 constexpr int kLinBM = 64;    // rows of A (tokens) per work-group
 constexpr int kLinBN = 64;    // rows of W (output features) per work-group, 16 per wave
+constexpr int kFewRows = 16;         // rows of A that few_linear_kernel takes
+constexpr int kFewWorkGroups = 256;  // its work-groups: one per CU
+constexpr int kFewStage = 512;       // bytes of a row of W per stage of a wave
 constexpr int kLinKC = 256;   // K elements per LDS chunk at 16-bit types (512 bytes; 128 at fp32)
 
 // Y = A W^T over the K range of one split; grid (splits, ceil(N/64), ceil(M/64)).
