@@ -602,3 +602,65 @@ def test_paged_prefill_rejects_bad_arguments():
     kc3 = torch.zeros((4, 12, 2, 64), dtype=torch.float16, device="cuda")
     with pytest.raises(RuntimeError, match="power of two"):
         flash_prefill_paged(q, kc3, kc3, table, 0)
+
+
+# ---- fp32 on split bf16 products (flash_prefill_f32.hip) -------------------------------
+
+def attend_visible(q, k, v, causal, scale=None):
+    """Float64 attention in which a key touches only the rows that see it."""
+    hq, hkv = q.shape[1], k.shape[1]
+    scale = q.shape[2] ** -0.5 if scale is None else scale
+    q, k, v = (t.double().cpu().numpy() for t in (q, k, v))
+    out = np.zeros(q.shape[:2] + v.shape[2:])
+    with np.errstate(invalid="ignore", over="ignore"):
+        for i in range(q.shape[0]):
+            n = min(i + 1, k.shape[0]) if causal else k.shape[0]
+            for h in range(hq):
+                s = k[:n, h // (hq // hkv)] @ q[i, h] * scale
+                e = np.exp(s - s.max())
+                out[i, h] = (e @ v[:n, h // (hq // hkv)]) / e.sum()
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,lq,lk,causal", [(2, 1, 1, 1, True), (8, 2, 33, 33, True), (3, 3, 64, 64, True),
+                                                 (4, 1, 97, 65, True), (2, 2, 130, 31, False), (1, 1, 70, 290, True),
+                                                 (8, 1, 1100, 1100, True), (40, 8, 800, 800, True)])   # one / two key groups
+def test_prefill_f32_split_products(d, hq, hkv, lq, lk, causal):
+    """Tile edges, rows and keys past the last tile, both key groupings.  A score's error is
+    a few roundings of the sum of its products' magnitudes; it moves a weight by as much, and
+    the output by twice that of the largest value."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    q, k, v = (randn(300 + i, n, h, d).cuda() for i, (n, h) in enumerate([(lq, hq), (lk, hkv), (lk, hkv)]))
+    out = flash_prefill_attention(q[None], k[None], v[None], causal)[0].double().cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(min(lq, 70)), np.arange(max(0, lq - 70), lq)]))
+    want = attend_visible(q, k, v, causal) if lq <= 200 else None
+    if want is None:
+        s = torch.einsum("qhd,khd->hqk", q[rows].double().cpu(), k.double().cpu().repeat_interleave(hq // hkv, 1))
+        s = s * d ** -0.5
+        if causal:
+            s.masked_fill_(torch.arange(lk)[None, None] > torch.from_numpy(rows)[None, :, None], -np.inf)
+        vv = v.double().cpu().repeat_interleave(hq // hkv, 1)
+        want, out = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), vv).numpy(), out[rows]
+    mag = float((q.abs().amax(1).amax(0) * k.abs().amax(1).amax(0)).sum()) * d ** -0.5
+    tol = (2 * 4 * mag + 8) * 2.0 ** -24 * float(v.abs().max())
+    assert np.abs(out - want).max() <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_f32_non_finite_values(d):
+    """Infinities, NaN and values near the fp32 limit reach the rows that see them and no other."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    n, hq, hkv = 150, 4, 2
+    q, k, v = (randn(310 + i, n, h, d).cuda() for i, h in enumerate([hq, hkv, hkv]))
+    v[40, 0, 3] = float("inf")
+    v[90, 0, 5] = float("nan")
+    v[20, 1, 7] = 3.4e38
+    k[120, 1, 2] = float("nan")
+    out = flash_prefill_attention(q[None], k[None], v[None])[0].double().cpu().numpy()
+    want = attend_visible(q, k, v, True)
+    assert np.array_equal(np.isnan(out), np.isnan(want)) and np.array_equal(np.isposinf(out), np.isposinf(want))
+    ok = np.isfinite(want)
+    assert (np.abs(out - want)[ok] <= 2e-5 * np.maximum(1.0, np.abs(want[ok]))).all()

@@ -435,6 +435,23 @@ def test_chunked_prefill_attends_to_prefix(dtype, dim, heads):
     assert max_err(own, want) < tol
 
 
+@pytest.mark.parametrize("dim,heads,kv_heads,rows", [(512, 8, 2, 200), (1024, 8, 8, 400)])    # head_dim 64, 128
+def test_f32_chunk_of_many_rows(dim, heads, kv_heads, rows):
+    """An fp32 chunk of enough rows reads its prefix through the block table in the prefill
+    kernel: its logits are those of one prefill of the whole prompt.  LOGIT_TOL is for the
+    128-wide model with weights of 0.05: a sum of `dim` products grows with sqrt(dim), and
+    with it q, k, the logits (std 6 at 1024) and every rounding, so the weights shrink by as
+    much."""
+    cfg = small_config(dim=dim, n_heads=heads, n_kv_heads=kv_heads, dtype="float32", max_seq_len=512)
+    model, kv, bm, ref, rk, rv = build(cfg, seed=9, std=0.05 * (128 / dim) ** 0.5, num_blocks=40)
+    toks = np.random.default_rng(26).integers(0, cfg.vocab_size, 45 + rows)
+    bm.register_sequence(0)
+    model.prefill(toks[:45], kv, bm, 0, logits=None)
+    got = model.prefill(toks[45:], kv, bm, 0, 45, attend_prefix=True)[0].cpu().numpy()
+    full = ref.prefill(toks, rk, rv, np.array(bm.get_block_table(0)), 0, 16)
+    assert max_err(got, full[45:]) < LOGIT_TOL["float32"]
+
+
 def prefill_batch(model, kv, bm, ref, rk, rv, lens, rng, cfg):
     """Prefill each sequence on both sides; returns the oracle's next tokens."""
     nxt = []

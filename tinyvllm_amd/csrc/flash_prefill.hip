@@ -15,8 +15,9 @@
 //    B-operand layout needed for O^T = V^T P^T once the two operands agree on
 //    the order of the reduction index, so P never leaves registers.
 //  * prefill_merge_kernel<D>: merges rows split into key chunks.
-//  * prefill_generic_kernel<T>: any D, Dv <= 256, any element type (fp32 path and
-//    odd head sizes).  One wave per (query row, head); 64 keys per step.
+//  * prefill_generic_kernel<T>: any D, Dv <= 256, any element type and alignment
+//    (odd head sizes; fp32 at head_dim 64 / 128 has flash_prefill_f32.hip).  One
+//    wave per (query row, head); 64 keys per step.
 #include "tv_common.h"
 #include "tv_paged_keys.h"
 #include "tv_params.h"
@@ -749,6 +750,10 @@ int launch_flash_prefill(const PrefillParams& p_in, int dtype, void* workspace, 
       if (d64) hipLaunchKernelGGL((prefill_merge_kernel<64>), mgrid, dim3(256), 0, stream, pp);
       else hipLaunchKernelGGL((prefill_merge_kernel<128>), mgrid, dim3(256), 0, stream, pp);
     }
+    return 0;
+  }
+  if (prefill_f32_supported(p_in, dtype)) {
+    launch_prefill_f32(p_in, stream);
     return 0;
   }
   if (p_in.head_dim > 256 || p_in.head_dim_v > 256) return 1;

@@ -20,6 +20,8 @@
 #include "../../include/tv_llama.h"
 #include "tv_dense.h"
 #include "tv_error.h"
+#include "tv_paged_keys.h"
+#include "tv_params.h"
 
 namespace {
 
@@ -240,6 +242,43 @@ int attend_fused(const tv_llama_model* m, const tv_llama_cache* c, const LayerIO
   return check_launch("step_attn");
 }
 
+// A chunk of an fp32 model over its cached prefix; false: no kernel for the shape.
+bool attend_prefix_f32(const tv_llama_model* m, const tv_llama_cache* c, const LayerIO& io, int l, float scale,
+                       hipStream_t s) {
+  const tv_llama_prefill_args* a = io.pargs;
+  const int bs = c->block_size;
+  const long long kv_len = (long long)a->start_pos + io.M;
+  // A row block walks the whole prefix whatever rows it has; with few rows and
+  // heads the paged decode of each row, which spreads over the CUs, is shorter.
+  // MI355X, two layers over 2040 cached tokens, rows paged / here: 32 heads of
+  // 128, 64 rows 1074 / 1144 us, 100 rows 2082 / 2020; 16 heads of 64, 64 rows
+  // 230 / 248, 100 rows 268 / 267; 32 heads of 64, 48 rows 398 / 389.
+  if ((long long)io.M * m->n_heads * 64 < 1536LL * m->head_dim) return false;
+  if ((bs & (bs - 1)) || (kv_len + bs - 1) / bs > tv::kPagedTableMax) return false;
+  tv::PrefillParams p{};
+  p.out = io.attn;
+  p.q = io.q;
+  p.k = c->k_caches[l];
+  p.v = c->v_caches[l];
+  p.q_len = io.M;
+  p.kv_len = (int)kv_len;
+  p.num_heads = m->n_heads;
+  p.num_kv_heads = m->n_kv_heads;
+  p.head_dim = p.head_dim_v = m->head_dim;
+  p.q_stride = p.out_stride = (long long)m->n_heads * m->head_dim;
+  p.k_stride = p.v_stride = (long long)m->n_kv_heads * m->head_dim;
+  p.causal = 1;
+  p.scale = scale;
+  p.out_dtype = TV_F32;
+  p.kv_table = a->block_table;
+  p.kv_num_blocks = c->num_blocks;
+  p.q_pos_offset = a->start_pos;
+  while ((1 << p.kv_bs_log2) < bs) ++p.kv_bs_log2;
+  if (!tv::prefill_f32_supported(p, TV_F32)) return false;
+  tv::launch_prefill_f32(p, s);
+  return true;
+}
+
 // The same without the fused kernel: qkv_rope, then tv_paged_decode (decode)
 // or tv_flash_prefill (prefill).  In the reference's order the decode stages
 // k/v with their slots and writes them after attention.
@@ -309,12 +348,13 @@ int attend_unfused(const tv_llama_model* m, const tv_llama_cache* c, const Layer
     // now, so the chunk attends keys 0 .. start_pos + M - 1 through the
     // sequence's table (MFMA tiles, causal at offset start_pos)
     const tv_llama_prefill_args* a = io.pargs;
+    if (dt == TV_F32 && attend_prefix_f32(m, c, io, l, scale, s)) return check_launch("attend_prefix_f32");
     rc = tv_flash_prefill_paged(io.attn, io.q, c->k_caches[l], c->v_caches[l], a->block_table, c->num_blocks,
                                 c->block_size, M, a->start_pos, m->n_heads, m->n_kv_heads, m->head_dim, qd, qd, 1,
                                 scale, dt, dt, s);
     if (rc == TV_EUNSUPPORTED) {
-      // fp32 models, odd head sizes or block sizes: row i is a paged decode of
-      // context start_pos + i + 1 over the sequence's one table row (stride 0)
+      // odd head sizes or block sizes: row i is a paged decode of context
+      // start_pos + i + 1 over the sequence's one table row (stride 0)
       const int width = a->bt_width * c->block_size;
       rc = tv_paged_decode(io.attn, io.q, c->k_caches[l], c->v_caches[l], a->block_table, io.slots, M, m->n_heads,
                            m->n_kv_heads, m->head_dim, c->block_size, c->num_blocks, 0, a->bt_width, scale, dt, dt,

@@ -98,6 +98,8 @@ bool launch_prefill_rows(const PrefillParams& p, int dtype, int num_seqs, int ma
 int launch_flash_prefill_paged(const PrefillParams& p, int dtype, hipStream_t stream);
 int launch_flash_prefill_varlen(const PrefillParams& p, int num_seqs, int max_q_len, int max_kv_len,
                                 long long total_q, int dtype, hipStream_t stream);
+bool prefill_f32_supported(const PrefillParams& p, int dtype);
+void launch_prefill_f32(const PrefillParams& p, hipStream_t stream);   // contiguous or paged (kv_table set) keys
 void launch_kv_write(const KVWriteParams& p, int vec_bytes, hipStream_t stream);
 void launch_kv_gather(const KVGatherParams& p, int vec_bytes, hipStream_t stream);
 
