@@ -188,6 +188,35 @@ def test_linear_few_rows(dtype, M, N, K, ks):
     check_products(dtype, M, N, K, ks)
 
 
+@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (64 + 33, 260, 96, 64), (129, 132, 1056, 352),   # 64 x 128 tiles
+                                      (321, 8260, 64, 64),                                            # several per CU
+                                      (300, 32000, 96, 96), (513, 16396, 32, 32)])                    # 128 x 128
+def test_linear_f32_many_rows(M, N, K, ks):
+    """fp32 products from split operands: tile edges, one and many stages, the three epilogues."""
+    check_products(torch.float32, M, N, K, ks)
+
+
+def test_linear_f32_many_rows_non_finite():
+    """Infinities, NaN and values beyond the largest bf16 give what fp32 products give."""
+    from tinyvllm_amd._lib import TV_F32
+    M, N, K = 70, 132, 64
+    a, w = gen(42, M, K, dtype=torch.float32), gen(43, N, K, dtype=torch.float32, scale=0.05)
+    a[3, 5], a[20, 7], a[66, 1] = float("inf"), float("nan"), 3.4e38
+    w[2, 9], w[131, 0] = float("-inf"), 3.4e38
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, N, K, 2, None, TV_F32, None), "logits")
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = f64(a) @ f64(w).T
+        want[np.abs(want) > 3.4028235e38] *= np.inf
+    got = f64(out)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    mag = np.abs(np.nan_to_num(f64(a), posinf=0)) @ np.abs(np.nan_to_num(f64(w), neginf=0)).T
+    assert (np.abs(got - want)[ok] <= 2e-5 * mag[ok]).all()
+
+
 def test_greedy_tie_resolves_to_first_index():
     """Two identical, dominant rows in different work-group tiles (5 and 70): every
     token ties between them and must take 5 (numpy / tinygrad argmax semantics)."""

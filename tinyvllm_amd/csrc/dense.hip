@@ -8,8 +8,8 @@
 //   greedy sampling  argmax over the vocabulary (first maximum)  sampling.py:131-134
 //
 // linear_kernel computes Y = A W^T for a skinny A (the decode batch, M <= 64
-// per work-group; at most 16 rows: few_linear_kernel; more than 64 at 16 bits:
-// tile_linear.hip) against a weight matrix W [N, K] that is streamed from HBM
+// per work-group; at most 16 rows: few_linear_kernel; more than 64:
+// tile_linear.hip, tile_linear_f32.hip) against a weight matrix W [N, K] that is streamed from HBM
 // exactly once.  Each of the 4 waves of a work-group owns 16 rows of W and all
 // 64 rows of A; A is staged in LDS per 512-byte-wide K chunk (256 fp16/bf16 or
 // 128 fp32 elements) and shared by the waves.  fp32 runs the same byte layout
@@ -404,6 +404,7 @@ template <typename T> static void launch_linear_t(const LinearParams& p, int epi
 
 void launch_linear(const LinearParams& p, int epi, int dtype, hipStream_t s) {
   if (tile_linear_supported(p, dtype)) return launch_tile_linear(p, epi, dtype, s);
+  if (dtype == kF32 && tile_linear_f32_supported(p)) return launch_tile_linear_f32(p, epi, s);
   if (dtype == kF16) launch_linear_t<_Float16>(p, epi, s);
   else if (dtype == kBF16) launch_linear_t<__bf16>(p, epi, s);
   else launch_linear_t<float>(p, epi, s);

@@ -3,10 +3,10 @@
 //
 // Same semantics as the other prefill kernels (flash_prefill.hip; reference
 // tinyvllm/model/llama.py:58-94).  An fp32 number is the exact sum of three
-// bf16 numbers of 8 bits each (split8), so a product of two is the sum of nine
-// bf16 products, each exact in fp32; the three smallest (2^-24 of the product
-// and below, of either sign) are left out.  Six v_mfma_f32_16x16x32_bf16 take
-// 96 cycles where eight v_mfma_f32_16x16x4_f32 take 256.
+// bf16 numbers of 8 bits each, so a product of two is the sum of nine bf16
+// products, each exact in fp32, of which the three smallest are left out
+// (tv_split.h).  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
+// v_mfma_f32_16x16x4_f32 take 256.
 //
 // A work-group owns 64 query rows of one head, 16 per wave; KS groups of four
 // waves share the row block's 32-key tiles (group s takes tiles s + KS j) and
@@ -22,6 +22,7 @@
 #include "tv_common.h"
 #include "tv_paged_keys.h"
 #include "tv_params.h"
+#include "tv_split.h"
 
 #include <algorithm>
 
@@ -31,38 +32,6 @@ namespace {
 
 constexpr int kBM = 64;   // query rows per work-group
 constexpr int kBN = 32;   // keys per tile
-
-// x = h + m + l with h, m, l in bf16: each rounds what the ones before leave,
-// and the last remainder has at most 8 bits.  (Finite x below the largest
-// bf16; beyond that the parts are not finite and the caller's result shows it.)
-__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  h = pack2<__bf16>(a, b);
-  a -= bf16_lo(h);
-  b -= bf16_hi(h);
-  m = pack2<__bf16>(a, b);
-  l = pack2<__bf16>(a - bf16_lo(m), b - bf16_hi(m));
-}
-__device__ __forceinline__ void split8(f32x4 a, f32x4 b, u32x4 (&s)[3]) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    uint32_t h, m, l;
-    split2(a[2 * i], a[2 * i + 1], h, m, l);
-    s[0][i] = h; s[1][i] = m; s[2][i] = l;
-    split2(b[2 * i], b[2 * i + 1], h, m, l);
-    s[0][2 + i] = h; s[1][2 + i] = m; s[2][2 + i] = l;
-  }
-}
-__device__ __forceinline__ f32x4 as_f32x4(u32x4 w) { return __builtin_bit_cast(f32x4, w); }
-
-// c += A B from the parts of both, smallest products first.
-__device__ __forceinline__ f32x4 mfma_split(const u32x4 (&a)[3], const u32x4 (&b)[3], f32x4 c) {
-  c = mfma16x16x32<__bf16>(a[2], b[0], c);
-  c = mfma16x16x32<__bf16>(a[0], b[2], c);
-  c = mfma16x16x32<__bf16>(a[1], b[1], c);
-  c = mfma16x16x32<__bf16>(a[1], b[0], c);
-  c = mfma16x16x32<__bf16>(a[0], b[1], c);
-  return mfma16x16x32<__bf16>(a[0], b[0], c);
-}
 
 // Element offset of key j's row in k / v.
 template <bool PAGED> __device__ __forceinline__ long long key_row(const PrefillParams& p, int j) {

@@ -67,7 +67,7 @@ int few_k_split(int N, int K, int es) {
 
 // K elements per split of a product whose consumer sums the partials.
 int k_split_of(int M, int N, int K, int dtype) {
-  if (M > tv::kLinBM && dtype != TV_F32) return tv::tile_linear_k_split(M, N, K);
+  if (M > tv::kLinBM) return dtype == TV_F32 ? tv::tile_linear_f32_k_split(M, N, K) : tv::tile_linear_k_split(M, N, K);
   if (M <= tv::kFewRows) return few_k_split(N, K, (int)elem_bytes(dtype));
   const long long full = round_up(K, 32);
   const long long tiles = ((N + tv::kLinBN - 1) / tv::kLinBN) * (long long)((M + tv::kLinBM - 1) / tv::kLinBM);

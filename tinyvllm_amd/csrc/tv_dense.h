@@ -102,6 +102,9 @@ void launch_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s
 // many-row products (tile_linear.hip)
 bool tile_linear_supported(const LinearParams& p, int dtype);
 int tile_linear_k_split(int M, int N, int K);
+bool tile_linear_f32_supported(const LinearParams& p);   // tile_linear_f32.hip
+int tile_linear_f32_k_split(int M, int N, int K);
+void launch_tile_linear_f32(const LinearParams& p, int epilogue, hipStream_t s);
 void launch_tile_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
 void launch_norm(const NormParams& p, int dtype, hipStream_t s);
 void launch_qkv_rope(const QKVParams& p, int dtype, hipStream_t s);
