@@ -664,3 +664,33 @@ def test_prefill_f32_non_finite_values(d):
     assert np.array_equal(np.isnan(out), np.isnan(want)) and np.array_equal(np.isposinf(out), np.isposinf(want))
     ok = np.isfinite(want)
     assert (np.abs(out - want)[ok] <= 2e-5 * np.maximum(1.0, np.abs(want[ok]))).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,start,bs", [(1000, 77, 16), (1024, 0, 4), (901, 640, 32)])
+def test_prefill_paged_128_row_kernel(dtype, n, start, bs):
+    """Grids of two 128-row work-groups per CU: prefixes and chunks that end inside a tile
+    and inside a block, small blocks, and an invalid block id, which makes NaN of the query
+    tiles that see it and of no other."""
+    from tinyvllm_amd.attention import flash_prefill_paged
+    hq, hkv, d = 64, 8, 128
+    total = start + n
+    nb = -(-total // bs) + 3
+    q, kc, vc = (randn(320 + i, *s, dtype=dtype).cuda()
+                 for i, s in enumerate([(n, hq, d), (nb, bs, hkv, d), (nb, bs, hkv, d)]))
+    table = torch.from_numpy(np.random.default_rng(5).permutation(nb)[:-(-total // bs)].astype(np.int32)).cuda()
+    out = flash_prefill_paged(q, kc, vc, table, start)[0].double().cpu()
+    k, v = (c[table.long()].reshape(-1, hkv, d)[:total].double().cpu() for c in (kc, vc))
+    rows = np.unique([0, 1, 31, 32, 127, 128, 500, n - 2, n - 1])
+    for h in (0, 7, 8, 63):
+        s = q[rows, h].double().cpu() @ k[:, h // 8].T.contiguous() / d ** 0.5
+        s.masked_fill_(torch.arange(total)[None] > torch.from_numpy(rows)[:, None] + start, -np.inf)
+        want = torch.softmax(s, -1) @ v[:, h // 8].contiguous()
+        assert (out[rows, h] - want).abs().max() < TOL[dtype]
+    bad = table.clone()
+    at = (start + 300) // bs                      # seen by the query tiles from row 300 - bs on
+    bad[at] = nb
+    out = flash_prefill_paged(q, kc, vc, bad, start)[0]
+    first = (at * bs - start) // 128 * 128        # first row of the first tile that sees the block
+    assert torch.isnan(out[first:]).all() and torch.isfinite(out[:first]).all()

@@ -764,6 +764,19 @@ int launch_flash_prefill(const PrefillParams& p_in, int dtype, void* workspace, 
   return 0;
 }
 
+// The 128-row kernel over a block table: where its grid gives every CU two
+// work-groups; below, the 64-row kernel's key groups are the shorter chain
+// (MI355X, bf16, Hkv 8, 64-row / 128-row kernel: Hq 32, 2048 rows after 100 /
+// 2048 / 6144 cached ones 70 / 63, 169 / 116, 370 / 252 us; 1500 after 1100
+// (384 work-groups) 76 / 77, 1024 after 2048 (256) 76 / 81).
+constexpr int kRowsPagedMinWorkGroups = 512;
+
+bool use_rows_kernel_paged(const PrefillParams& p) {
+  return p.head_dim == 128 && (long long)p.num_heads * ((p.q_len + 127) / 128) >= kRowsPagedMinWorkGroups &&
+         p.kv_bs_log2 >= 2 &&
+         ((long long)p.kv_len + (1LL << p.kv_bs_log2) - 1) >> p.kv_bs_log2 <= kRowsTableMax;
+}
+
 // One prompt whose keys and values are read through a block table
 // (kv_table set) with query rows at positions q_pos_offset ..: the 64-row
 // kernel with its loads going through the table.  Returns 1 when the shape has
@@ -775,6 +788,7 @@ int launch_flash_prefill_paged(const PrefillParams& p_in, int dtype, hipStream_t
   if (((long long)pp.kv_len + (1LL << pp.kv_bs_log2) - 1) >> pp.kv_bs_log2 > kPagedTableMax) return 1;
   pp.xcd_remap = (pp.num_heads % 8 == 0) ? 1 : 0;
   pp.chunk_tiles = 1 << 20;
+  if (use_rows_kernel_paged(pp) && launch_prefill_rows(pp, dtype, 1, pp.q_len, nullptr, stream)) return 0;
   int units, max_chunks;
   prefill_units(pp, units, max_chunks);
   pp.max_chunks = 1;

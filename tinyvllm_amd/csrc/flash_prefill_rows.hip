@@ -115,7 +115,13 @@ __host__ __device__ constexpr bool rows_split_f32(int out_dtype) {
   return out_dtype == kF32 || !std::is_same_v<T, _Float16>;
 }
 
-template <typename T, int D>
+// PAGED: keys and values are read through p.kv_table, the query rows start at
+// position p.q_pos_offset.  A DMA instruction's 1 KB are four tile rows, which
+// lie in one block of four rows or more, so it takes a descriptor of its own at
+// the block's row; the block ids are staged in LDS.  MI355X, Llama-3-8B heads,
+// bf16, a chunk of 2048 rows after 2048 cached ones: 116 us (890 TFLOP/s), the
+// 64-row kernel 169.
+template <typename T, int D, bool PAGED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_rows_kernel(const PrefillParams pa) {
   PrefillParams p = pa;
@@ -143,6 +149,8 @@ prefill_rows_kernel(const PrefillParams pa) {
   constexpr int SPR = ROWB / 16;           // 16-byte chunks per row
   static_assert(NI >= 1 && NI * 4 * 1024 == TILEB, "tile / DMA shape");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NB * BUFB];
+  __shared__ int stbl[PAGED ? kRowsTableMax : 1];
+  __shared__ int sbad;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -157,7 +165,8 @@ prefill_rows_kernel(const PrefillParams pa) {
   const int kvh = h / (p.num_heads / p.num_kv_heads);
   const int klim = p.kv_len;
   int kbeg, kend;          // this unit's keys
-  rows_unit_keys(qt, half, p.causal ? min(klim, (qt + 1) * BM) : klim, kbeg, kend);
+  const int qoff = PAGED ? p.q_pos_offset : 0;
+  rows_unit_keys(qt, half, p.causal ? min(klim, (qt + 1) * BM + qoff) : klim, kbeg, kend);
   const int ntiles = (kend - kbeg + BN - 1) / BN;
   const float c = p.scale * kLog2e;
   const int row0 = qt * BM + wave * 32;    // first query row of this wave
@@ -192,8 +201,9 @@ prefill_rows_kernel(const PrefillParams pa) {
     const int row = (wave * NI + i) * RPI + lane / SPR;
     const int slot = lane % SPR;
     const int chunk = slot ^ tile_chunk_perm<D>(row);
-    kvoff[i] = (uint32_t)(row * kstr + chunk * 16);
-    vvoff[i] = (uint32_t)(row * vstr + chunk * 16);
+    const int brow = PAGED ? lane / SPR : row;      // from the descriptor's base
+    kvoff[i] = (uint32_t)(brow * kstr + chunk * 16);
+    vvoff[i] = (uint32_t)(brow * vstr + chunk * 16);
   }
   // Tile t (keys kbeg + 32 t ..) into buffer t % NB.  Its K / V buffer
   // descriptors: base at the tile's first key row, range ending at the last
@@ -207,7 +217,34 @@ prefill_rows_kernel(const PrefillParams pa) {
   unsigned long long vr = (unsigned long long)(klim - 1 - kbeg) * vstr + D * sizeof(T);
   const unsigned long long kstep = (unsigned long long)BN * kstr;
   const unsigned long long vstep = (unsigned long long)BN * vstr;
+  const int lg = p.kv_bs_log2;
+  const int kpad = min(klim, (kend + 2 * BN - 1) / BN * BN);   // end of the keys that are requested
+  bool bad = false;
+  int nextid[NI];          // block ids of the next request
+  auto request_key = [&](int t, int i) {
+    return min(min(t, ntiles - 1) * BN + (wave * NI + i) * RPI, kpad - 1);
+  };
   auto issue = [&](int t) {
+    const uint32_t buf = lds0 + (uint32_t)((t % NB) * BUFB);
+    if constexpr (PAGED) {
+      u32x4 rk[NI], rv[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int key = min(t, ntiles - 1) * BN + (wave * NI + i) * RPI;
+        const int rows = min(RPI, kpad - key);      // keys past the last: zeros
+        const unsigned long long row =
+            ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(nextid[i]) << lg) + (key & ((1 << lg) - 1));
+        rk[i] = rsrc_words(kbase + row * kstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)kstr + ROWB) : 0);
+        rv[i] = rsrc_words(vbase + row * vstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)vstr + ROWB) : 0);
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) load_lds16(rk[i], sgpr(buf + (uint32_t)((wave * NI + i) * 1024)), kvoff[i]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) load_lds16(rv[i], sgpr(buf + (uint32_t)(TILEB + (wave * NI + i) * 1024)), vvoff[i]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) nextid[i] = stbl[request_key(t + 1, i) >> lg];
+      return;
+    }
     if (t > 0 && t < ntiles) {
       ka += kstep;
       kr -= kstep;
@@ -216,7 +253,6 @@ prefill_rows_kernel(const PrefillParams pa) {
     }
     const u32x4 rk = rsrc_words(reinterpret_cast<const void*>(ka), kr);
     const u32x4 rv = rsrc_words(reinterpret_cast<const void*>(va), vr);
-    const uint32_t buf = lds0 + (uint32_t)((t % NB) * BUFB);
 #pragma unroll
     for (int i = 0; i < NI; ++i) load_lds16(rk, sgpr(buf + (uint32_t)((wave * NI + i) * 1024)), kvoff[i]);
 #pragma unroll
@@ -226,11 +262,26 @@ prefill_rows_kernel(const PrefillParams pa) {
   // The Q loads are the only global loads the compiler tracks; retire them
   // here so its own wait for them cannot land inside the tile loop (where it
   // would also drain the LDS-DMA loads in flight).
+  if constexpr (PAGED) {   // an invalid id reads block 0 (in bounds) and makes the rows NaN
+    if (threadIdx.x == 0) sbad = 0;
+    lds_barrier();
+    for (int i = threadIdx.x; i <= (kpad - 1) >> lg; i += 256) {
+      const int b = p.kv_table[i];
+      const bool ok = (unsigned)b < (unsigned)p.kv_num_blocks;
+      stbl[i] = ok ? b : 0;
+      if (!ok && i <= (kend - 1) >> lg) sbad = 1;
+    }
+  }
   wait_vmcnt<0>();
   // Rows past kv_len read as zero through the resource range; the buffers start
   // zeroed so nothing non-finite can reach a masked product.
   for (int i = threadIdx.x; i < NB * BUFB / 16; i += 256) reinterpret_cast<u32x4*>(smem)[i] = u32x4{0, 0, 0, 0};
   lds_barrier();
+  if constexpr (PAGED) {
+    bad = sbad != 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) nextid[i] = stbl[request_key(0, i) >> lg];
+  }
   issue(0);
   issue(1);
 
@@ -277,10 +328,10 @@ prefill_rows_kernel(const PrefillParams pa) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) st[r][kb][i] = fmaf(st[r][kb][i], c, -mref[r]);
     }
-    if (!(k0 + 16 * NKB <= kend && (!p.causal || k0 + 16 * NKB - 1 <= row0))) {
+    if (!(k0 + 16 * NKB <= kend && (!p.causal || k0 + 16 * NKB - 1 <= row0 + qoff))) {
 #pragma unroll
       for (int r = 0; r < RB; ++r) {
-        const int rel = (p.causal ? min(kend - 1, qi[r]) : kend - 1) - (k0 + 4 * g);
+        const int rel = (p.causal ? min(kend - 1, qi[r] + qoff) : kend - 1) - (k0 + 4 * g);
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
@@ -337,7 +388,7 @@ prefill_rows_kernel(const PrefillParams pa) {
     issue(jj + 2);
     issue(jj + 3);
     const int k0 = kbeg + jj * BN;
-    if (idle || (p.causal && k0 > row0 + 31)) return;
+    if (idle || (p.causal && k0 > row0 + 31 + qoff)) return;
     f32x4 st[RB][2 * KB];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
@@ -411,7 +462,11 @@ prefill_rows_kernel(const PrefillParams pa) {
     for (int db = 0; db < DB; ++db) {
       const size_t idx = (half >= 0 ? hrow * D : (size_t)qi[r] * p.out_stride + (size_t)h * D) + db * 16 + 4 * g;
       const f32x4 v = oacc[r][db] * inv;
-      if (f32rows) {
+      if (PAGED && bad) {      // integer stores: this file is compiled without NaN semantics
+        if (f32rows) *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(obase) + idx) = u32x4{0x7FC00000u, 0x7FC00000u, 0x7FC00000u, 0x7FC00000u};
+        else *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(obase) + idx) =
+            ElemTraits<T>::kCode == kF16 ? u32x2{0x7E007E00u, 0x7E007E00u} : u32x2{0x7FC07FC0u, 0x7FC07FC0u};
+      } else if (f32rows) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(obase) + idx) = v;
       } else {
         const u32x2 w = u32x2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
@@ -491,7 +546,7 @@ __global__ void __launch_bounds__(256) prefill_rows_merge_kernel(const PrefillPa
 template <typename T, int D>
 long long rows_resident() {
   static std::atomic<long long> slots[kMaxDevices];
-  return resident_work_groups(slots, prefill_rows_kernel<T, D>, 256);
+  return resident_work_groups(slots, prefill_rows_kernel<T, D, false>, 256);
 }
 
 // First split query tile (rows_split) of a launch; nqt: no split.  One causal
@@ -552,7 +607,7 @@ void launch_rows(const PrefillParams& pp_in, int num_seqs, int max_q_len, void* 
     pp.split_o = workspace;
     pp.split_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + ml_offset);
     pp.longest_first = 0;
-    hipLaunchKernelGGL((prefill_rows_kernel<T, D>), dim3(pp.num_heads, 2 * nqt - pp.rows_split), dim3(256), 0,
+    hipLaunchKernelGGL((prefill_rows_kernel<T, D, false>), dim3(pp.num_heads, 2 * nqt - pp.rows_split), dim3(256), 0,
                        stream, pp);
     const dim3 mgrid(pp.num_heads, nqt - pp.rows_split, kRowsMergeParts);
     using H = std::conditional_t<rows_split_f32<T>(ElemTraits<T>::kCode), float, T>;   // halves of a T output
@@ -564,7 +619,8 @@ void launch_rows(const PrefillParams& pp_in, int num_seqs, int max_q_len, void* 
   }
   const dim3 grid(pp.num_heads, nqt, num_seqs);
   pp.longest_first = (long long)grid.x * grid.y * grid.z > rows_resident<T, D>() ? 1 : 0;
-  hipLaunchKernelGGL((prefill_rows_kernel<T, D>), grid, dim3(256), 0, stream, pp);
+  if (pp.kv_table) hipLaunchKernelGGL((prefill_rows_kernel<T, D, true>), grid, dim3(256), 0, stream, pp);
+  else hipLaunchKernelGGL((prefill_rows_kernel<T, D, false>), grid, dim3(256), 0, stream, pp);
 }
 
 // Workspace of a one-prompt launch (0: no split, or a shape not handled here).

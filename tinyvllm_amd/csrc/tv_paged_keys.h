@@ -17,6 +17,8 @@ namespace tv {
 
 // Block ids a paged work-group can stage (keys of 65536 tokens at block size 16).
 constexpr int kPagedTableMax = 4096;
+// The same for the 128-row kernel (two work-groups per CU beside their tiles).
+constexpr int kRowsTableMax = 2048;
 
 // End of a query tile's key range: causal rows see keys j <= i + q_pos_offset.
 __host__ __device__ inline int prefill_unit_key_end(bool causal, int klim, int qt, int rows, int q_pos_offset) {
