@@ -251,12 +251,13 @@ __global__ void __launch_bounds__(256, kLinearMinBlocks) linear_kernel(const Lin
 // logits, whose argmax keys cover 64 features).  One work-group per CU walks
 // the units; its loads run ahead across them.  The 64-row kernel spent its
 // time on products for rows that are not there (fp32) and on one 64-row tile
-// per work-group, 176 of them on 256 CUs.  MI355X, 4 rows, against it:
-// 11264 x 2048 fp32 47 -> 20.0 us (4.6 TB/s), 32000 x 2048 87 -> 47.7 (5.5),
-// 2048 x 5632 26 -> 12.5; fp16 15.9 -> 11.3, 31.4 -> 24.9, 9.4 -> 7.3.  At 16
-// rows, fp16: 16.4 -> 13.5, 31.7 -> 26.3, 9.9 -> 8.6.  Rejected: A held in LDS
-// with W in registers (fp32 25.9 / 62.9 / 12.6 us), both in registers (29.1 /
-// 56.0 / 13.8); there an instruction reads 64 bytes of 16 rows.
+// per work-group, 176 of them on 256 CUs.  W is read once and non-temporally
+// (32000 x 2048 fp32 48.4 us without, 43.7 with).  MI355X, 4 rows, against the
+// 64-row kernel: 11264 x 2048 fp32 47 -> 19.0 us (4.9 TB/s), 32000 x 2048 87 ->
+// 43.7 (6.0), 2048 x 5632 26 -> 11.5; fp16 15.9 -> 10.8, 31.4 -> 22.7, 9.4 ->
+// 7.0.  At 16 rows, fp16: 16.4 -> 12.7, 31.7 -> 24.5, 9.9 -> 8.1.  Rejected: A
+// held in LDS with W in registers (fp32 25.9 / 62.9 / 12.6 us), both in
+// registers (29.1 / 56.0 / 13.8); there an instruction reads 64 bytes of 16 rows.
 template <typename T, int EPI, int KW, int RA, int S>
 __global__ void __launch_bounds__(256) few_linear_kernel(const LinearParams p) {
   constexpr int ES = (int)sizeof(T);
@@ -328,7 +329,7 @@ __global__ void __launch_bounds__(256) few_linear_kernel(const LinearParams p) {
     for (int t = 0; t < LW; ++t) {
       const int r = 2 * t + lrow, o = 16 * ((lane & 31) ^ r);
       const bool in = o < left && r < src.rows_w;
-      load_lds16(src.wres, base + t * 1024, in ? (uint32_t)(r * p.K * ES + c * CB + o) : 0x80000000u);
+      load_lds16_nt(src.wres, base + t * 1024, in ? (uint32_t)(r * p.K * ES + c * CB + o) : 0x80000000u);
     }
 #pragma unroll
     for (int t = 0; t < LA; ++t) {

@@ -28,6 +28,14 @@ __device__ __forceinline__ void load_lds16(u32x4 rsrc, uint32_t lds_base, uint32
                : "memory", "m0");
 }
 
+// The same for lines that are read once (non-temporal).
+__device__ __forceinline__ void load_lds16_nt(u32x4 rsrc, uint32_t lds_base, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds"
+               :
+               : "s"(lds_base), "v"(voff), "s"(rsrc)
+               : "memory", "m0");
+}
+
 // Wait until at most N vector-memory operations of this wave are outstanding
 // (gfx9 s_waitcnt: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]).
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
