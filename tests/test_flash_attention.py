@@ -6,6 +6,8 @@ MFMA-path parity for fp16/bf16 at the benchmark shapes.
 Tolerances (max-abs vs the float64 oracle): fp32 1e-4, fp16/bf16 2e-2.
 """
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -694,3 +696,34 @@ def test_prefill_paged_128_row_kernel(dtype, n, start, bs):
     out = flash_prefill_paged(q, kc, vc, bad, start)[0]
     first = (at * bs - start) // 128 * 128        # first row of the first tile that sees the block
     assert torch.isnan(out[first:]).all() and torch.isfinite(out[:first]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_prefill_paged_128_row_kernel_divides_by_the_rounded_weights(dtype):
+    """A weight is rounded to the input type on its way into P V; the row sum has to hold the
+    rounded ones, so that the rounding cancels where one key dominates.  Here a weight w = 2^t,
+    t in 6.5 .. 7.6 above a key of weight one and value zero, meets one value: the output is
+    v w / (w + 1), and a relative error e of w (its rounding of 2^-9 at most, at fp16 the
+    2^-11 t of the scaled queries) moves it by e / (w + 1), 7e-5 at most.  A sum of unrounded
+    weights is off by the rounding itself, up to 2e-3 (bf16) and 4e-4 (fp16)."""
+    from tinyvllm_amd.attention import flash_prefill_paged
+    hq, hkv, d, n, start, bs = 64, 8, 128, 1000, 77, 16
+    total = start + n
+    nb = -(-total // bs)
+    t = torch.linspace(6.5, 7.6, n * hq, dtype=torch.float64).reshape(n, hq)
+    q = torch.zeros((n, hq, d), dtype=torch.float64)
+    q[:, :, 0] = t / math.log2(math.e) * d ** 0.5 / 16
+    k = torch.zeros((nb * bs, hkv, d), dtype=torch.float64)
+    k[1:, :, 0], k[70, :, 0] = -64, 16
+    v = torch.zeros((nb * bs, hkv, d), dtype=torch.float64)
+    v[70] = randn(330, hkv, d).double()
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    table = torch.from_numpy(np.random.default_rng(6).permutation(nb).astype(np.int32))
+    kc, vc = (torch.empty((nb, bs, hkv, d), dtype=dtype) for _ in range(2))
+    kc[table.long()], vc[table.long()] = k.view(nb, bs, hkv, d), v.view(nb, bs, hkv, d)
+    out = flash_prefill_paged(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(), start, out_dtype=torch.float32)[0]
+    out = out.double().cpu()
+    w = torch.exp(q[:, :, 0].double() * 16 / d ** 0.5)
+    want = v[70].double().repeat_interleave(hq // hkv, 0) * (w / (w + 1))[:, :, None]
+    assert ((out - want).abs() <= 1e-4 * want.abs()).all()

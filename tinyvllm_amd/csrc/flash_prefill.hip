@@ -119,10 +119,6 @@ __device__ __forceinline__ void store4(void* base, size_t idx, f32x4 v, int out_
 // and loaded two steps ahead through buffer loads whose range ends at the last
 // key row (rows past kv_len read as zero), one barrier per step.
 
-template <typename T> constexpr uint32_t kOnes2 = 0;
-template <> constexpr uint32_t kOnes2<_Float16> = 0x3C003C00u;
-template <> constexpr uint32_t kOnes2<__bf16> = 0x3F803F80u;
-
 // maximum of the 4 KB values of one S^T tile (v_max3 tree)
 template <int KB> __device__ __forceinline__ float max_tile(const f32x4 (&st)[KB]) {
   float t[KB];

@@ -35,7 +35,14 @@
 // rounding to T for the P V product) and are summed over the four lanes of a
 // query at the end.  v_dot2 against ones on the packed P cannot issue beside
 // the wave's in-flight MFMAs on gfx950; the adds can, and measured 2-3.5%
-// faster at L 2048 / 8192 (1.5% slower at 4096).
+// faster at L 2048 / 8192 (1.5% slower at 4096).  A chunk over a block table
+// sums the rounded weights instead (one MFMA of P against ones per 32 keys), as
+// the 64-row kernel does for the chunks of smaller grids: a weight's rounding
+// then cancels where it dominates its row.  Error of the output against 64 bits
+// (2-norm; 2048 rows after 2048 cached ones, scores of standard deviation 1 /
+// 3): bf16 2.34e-3 / 1.97e-3, 2.35e-3 / 2.16e-3 with unrounded sums and 2.34e-3
+// / 1.95e-3 in the 64-row kernel; fp16 3.61e-4 / 4.99e-4, 3.61e-4 / 5.10e-4 and
+// 3.61e-4 / 4.97e-4.  The time of the chunk's pass did not move (1062 us).
 //
 // Measured on MI355X (Llama-3-8B heads, Hq 32 / Hkv 8, head_dim 128, fp16,
 // causal): L 2048 54-56 us (51 us replayed in a graph) against 64-68 for the
@@ -303,6 +310,7 @@ prefill_rows_kernel(const PrefillParams pa) {
 
   f32x4 oacc[RB][DB];
   float lpart[RB];      // this lane's share of the row sum (keys 4g..4g+3 of every 16)
+  f32x4 lones[RB];      // PAGED: the row sum in element 0 (ones x P; the other elements are not kept)
   float mref[RB], thr[RB];
   f32x4 negm[RB];       // -m in every element: the fp16 score accumulator's initial value
 #pragma unroll
@@ -310,6 +318,7 @@ prefill_rows_kernel(const PrefillParams pa) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) oacc[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
     lpart[r] = 0.0f;
+    lones[r] = f32x4{0.f, 0.f, 0.f, 0.f};
     mref[r] = 0.0f;
     thr[r] = -__FLT_MAX__;
     negm[r] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -360,7 +369,8 @@ prefill_rows_kernel(const PrefillParams pa) {
         const float alpha = need && thr[r] > 0.0f ? fast_exp2(-delta) : 1.0f;
 #pragma unroll
         for (int db = 0; db < DB; ++db) oacc[r][db] *= alpha;
-        lpart[r] *= alpha;
+        if constexpr (PAGED) lones[r][0] *= alpha;
+        else lpart[r] *= alpha;
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) st[r][kb] -= delta;
         mref[r] += delta;
@@ -433,7 +443,10 @@ prefill_rows_kernel(const PrefillParams pa) {
         const u32x4 pf = u32x4{pack2<T>(e[0], e[1]), pack2<T>(e[2], e[3]), pack2<T>(e[4], e[5]), pack2<T>(e[6], e[7])};
 #pragma unroll
         for (int db = 0; db < DB; ++db) oacc[r][db] = mfma16x16x32<T>(vf[db], pf, oacc[r][db]);
-        lpart[r] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+        if constexpr (PAGED)
+          lones[r] = mfma16x16x32<T>(u32x4{kOnes2<T>, kOnes2<T>, kOnes2<T>, kOnes2<T>}, pf, lones[r]);
+        else
+          lpart[r] += ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
       }
     }
   };
@@ -453,7 +466,7 @@ prefill_rows_kernel(const PrefillParams pa) {
   const bool f32rows = half >= 0 ? rows_split_f32<T>(p.out_dtype) : p.out_dtype == kF32;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
-    const float lsum = sum_over_g(lpart[r]);
+    const float lsum = PAGED ? lones[r][0] : sum_over_g(lpart[r]);
     if (qi[r] >= p.q_len) continue;
     const float inv = 1.0f / lsum;
     const size_t hrow = (sunit * 2 + (half > 0)) * BM + (qi[r] - qt * BM);   // row of a half

@@ -28,6 +28,11 @@ template <> struct ElemTraits<float> { static constexpr int kCode = kF32; };
 template <> struct ElemTraits<_Float16> { static constexpr int kCode = kF16; };
 template <> struct ElemTraits<__bf16> { static constexpr int kCode = kBF16; };
 
+// two ones, packed
+template <typename T> inline constexpr uint32_t kOnes2 = 0;
+template <> inline constexpr uint32_t kOnes2<_Float16> = 0x3C003C00u;
+template <> inline constexpr uint32_t kOnes2<__bf16> = 0x3F803F80u;
+
 // ---- conversions on packed 32-bit words -----------------------------------
 
 // Reinterpret a 32-bit word as float.  Takes the word by value: applying
