@@ -652,6 +652,21 @@ def test_prefill_f32_split_products(d, hq, hkv, lq, lk, causal):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
+def test_prefill_f32_positive_sums(d):
+    """Equal weights over 32768 positive values: the sum of a key group's 512 (or 256) tiles
+    walks by at most 2^-24 of it per tile, about sqrt(512) 2^-24 = 1.3e-6 in the end; the row sum
+    is exact.  (Low parts added to the whole sum one by one: 1e-5 and above.)"""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    q = torch.zeros((1, 64, 2, d), device="cuda")
+    k = randn(340, 1, 32768, 1, d).cuda()
+    v = torch.rand((1, 32768, 1, d), generator=torch.Generator().manual_seed(341)).cuda()
+    out = flash_prefill_attention(q, k, v, False)
+    want = v[0, :, 0].double().mean(0)
+    assert ((out.double() - want).norm() / want.norm() / (64 * 2) ** 0.5).item() < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
 def test_prefill_f32_non_finite_values(d):
     """Infinities, NaN and values near the fp32 limit reach the rows that see them and no other."""
     from tinyvllm_amd.attention import flash_prefill_attention

@@ -196,6 +196,23 @@ def test_linear_f32_many_rows(M, N, K, ks):
     check_products(torch.float32, M, N, K, ks)
 
 
+@pytest.mark.parametrize("M,N", [(70, 260), (512, 8260)])       # 64 x 128, 128 x 128 tiles
+def test_linear_f32_many_rows_positive_sums(M, N):
+    """Sums of 16384 positive products: 512 stages, each rounded into the sum by 2^-24 of it at
+    most and without a bias, so the error walks to about sqrt(512) 2^-24 = 1.3e-6 of the sum.
+    (Low parts added to the whole sum one by one are lost once it is 2^8 products long, always
+    with the same sign: 1.8e-5.)"""
+    from tinyvllm_amd._lib import TV_F32
+    K = 16384
+    g = torch.Generator().manual_seed(44)
+    a, w = (torch.rand((n, K), generator=g).cuda() for n in (M, N))
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, N, K, 2, None, TV_F32, None), "logits")
+    torch.cuda.synchronize()
+    want = a.double() @ w.double().T.contiguous()
+    assert ((out.double() - want).norm() / want.norm()).item() < 2e-6
+
+
 def test_linear_f32_many_rows_non_finite():
     """Infinities, NaN and values beyond the largest bf16 give what fp32 products give."""
     from tinyvllm_amd._lib import TV_F32

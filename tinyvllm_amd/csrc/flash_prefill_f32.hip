@@ -269,7 +269,7 @@ prefill_f32_kernel(const PrefillParams p) {
         const u32x2 hi = lds_read_tr16(a + 16 * KP);
         vf[q] = u32x4{lo[0], lo[1], hi[0], hi[1]};
       }
-      oacc[db] = mfma_split(vf, pf, oacc[db]);
+      oacc[db] += mfma_split(vf, pf, f32x4{0.f, 0.f, 0.f, 0.f});   // one fp32 add per tile (tile_linear_f32.hip)
     }
   };
 

@@ -154,11 +154,17 @@ tile_linear_f32_kernel(const LinearParams p) {
       u32x4 fw[3];
 #pragma unroll
       for (int q = 0; q < 3; ++q) fw[q] = *reinterpret_cast<const u32x4*>(lds + fw_at[nb] + q * PLANE);
+      // A stage's products start from zero and join the sum in one fp32 add:
+      // added one by one, the small ones would fall below the rounding of a sum
+      // of many stages, and as they have the sign of the product, never cancel.
+      f32x4 part[MBW];
 #pragma unroll
       for (int q = 0; q < kSplitProducts; ++q)
 #pragma unroll
         for (int mb = 0; mb < MBW; ++mb)
-          acc[mb][nb] = mfma16x16x32<__bf16>(fw[kSplitA[q]], fa[mb][kSplitB[q]], acc[mb][nb]);
+          part[mb] = mfma16x16x32<__bf16>(fw[kSplitA[q]], fa[mb][kSplitB[q]], q ? part[mb] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int mb = 0; mb < MBW; ++mb) acc[mb][nb] += part[mb];
     }
   }
 
