@@ -213,6 +213,37 @@ def test_linear_f32_many_rows_positive_sums(M, N):
     assert ((out.double() - want).norm() / want.norm()).item() < 2e-6
 
 
+@pytest.mark.parametrize("low_bits", [False, True])
+@pytest.mark.parametrize("terms", [1, 32])
+def test_linear_f32_many_rows_parts(low_bits, terms):
+    """Every part product counts, and none is one-sided: outputs of one product each, and sums
+    of 32 products of one sign, with random significands or with all low bits set.  The products
+    left out are at most 2^-24 of the whole; six products are added smallest first, so one
+    rounding of 2^-24 and parts of 2^-8 of it follow.  A lost part product is 2^-17 or more,
+    parts that are cut off leave 8 * 2^-24."""
+    from tinyvllm_amd._lib import TV_F32
+    M, N, K = 96, 260, 32
+    rng = np.random.default_rng(45)
+
+    def draw(*shape):
+        bits = rng.integers(0, 1 << 23, shape) | 0x3f800000
+        if low_bits:
+            bits |= 0xffff
+        return torch.from_numpy(bits.astype(np.int32)).view(torch.float32)
+
+    a, w = draw(M, K), draw(N, K)
+    if terms == 1:
+        a = a * torch.nn.functional.one_hot(torch.arange(M) % K, K)
+        a *= torch.from_numpy(2.0 ** rng.integers(-20, 20, (M, 1))).float()
+        w[::2] *= -1
+    a, w = a.cuda(), w.cuda()
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, N, K, 2, None, TV_F32, None), "logits")
+    torch.cuda.synchronize()
+    want = a.double() @ w.double().T.contiguous()
+    assert ((out.double() - want).abs() <= 2.5 * 2.0 ** -24 * want.abs()).all()
+
+
 def test_linear_f32_many_rows_non_finite():
     """Infinities, NaN and values beyond the largest bf16 give what fp32 products give."""
     from tinyvllm_amd._lib import TV_F32

@@ -3,10 +3,11 @@
 //
 // Same semantics as the other prefill kernels (flash_prefill.hip; reference
 // tinyvllm/model/llama.py:58-94).  An fp32 number is the exact sum of three
-// bf16 numbers of 8 bits each, so a product of two is the sum of nine bf16
-// products, each exact in fp32, of which the three smallest are left out
-// (tv_split.h).  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
-// v_mfma_f32_16x16x4_f32 take 256.
+// bf16 numbers, so a product of two is the sum of nine bf16 products, each
+// exact in fp32, of which the three smallest are left out (tv_split.h).  Six
+// v_mfma_f32_16x16x32_bf16 take 96 cycles where eight v_mfma_f32_16x16x4_f32
+// take 256.  Every chain of six starts from zero and joins the score or the
+// output in one fp32 add (tile_linear_f32.hip).
 //
 // A work-group owns 64 query rows of one head, 16 per wave; KS groups of four
 // waves share the row block's 32-key tiles (group s takes tiles s + KS j) and
@@ -17,8 +18,11 @@
 // The split costs about as many issue slots per tile as the products, so
 // neither unit is full; two work-groups (or key groups) per CU overlap them.
 // MI355X, causal, against one wave per query row on the VALU: Hq 32 / Hkv 4,
-// head_dim 64: L 64 8.9 -> 5.9 us, L 512 178 -> 18, L 1500 1347 -> 70; Hkv 8,
-// head_dim 128: L 512 357 -> 30, L 1500 2834 -> 144 (128 TFLOP/s of attention).
+// head_dim 64: L 64 8.9 -> 6.0 us, L 512 174 -> 18, L 1500 1347 -> 71; Hkv 8,
+// head_dim 128: L 512 354 -> 31, L 1500 2834 -> 150 (123 TFLOP/s of attention).
+// Error against 64 bits (2-norm; L 64 / 300 / 700): N(0, 1) 0.8e-7 / 1.1e-7 /
+// 1.1e-7, the VALU kernel 1.8e-7 / 3.1e-7 / 3.0e-7; scores of standard deviation
+// 6: 1.9e-7 / 2.8e-7 / 3.0e-7 against 4.7e-7 / 9.8e-7 / 8.3e-7.
 #include "tv_common.h"
 #include "tv_paged_keys.h"
 #include "tv_params.h"
@@ -223,7 +227,7 @@ prefill_f32_kernel(const PrefillParams p) {
 #pragma unroll
         for (int q = 0; q < 3; ++q)
           kf[q] = *reinterpret_cast<const u32x4*>(tile + q * PLANE + (kb * 16 + col) * KP + ks * 32 + g * 8);
-        s[kb] = mfma_split(kf, qf[ks], s[kb]);
+        s[kb] += mfma_split(kf, qf[ks], f32x4{0.f, 0.f, 0.f, 0.f});
       }
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)

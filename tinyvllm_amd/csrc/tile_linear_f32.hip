@@ -10,15 +10,20 @@
 // so fragment reads and writes touch every bank once.
 //
 // What bounds it: the matrix unit at the rate it sustains (512 x 32000 x 2048:
-// 372 us, 1.08 PFLOP/s of bf16; the 16-bit product reaches 1.23), and below
+// 365 us, 1.10 PFLOP/s of bf16; the 16-bit product reaches 1.23), and below
 // that size the split, which takes its issue slots (64 x 128 tile: 528 clocks
 // of a stage beside 768 of products).  Four work-groups per CU of the smaller
-// tile (114 registers) run their splits beside each other's products; two with
+// tile (118 registers) run their splits beside each other's products; two with
 // a second stage buffer, split and products interleaved, were 3% slower.
-// MI355X, against fp32 products on the skinny kernel: 300 x 11264 x 2048 160 ->
-// 117 us, 300 x 2048 x 5632 85 -> 55, 512 x 32000 x 2048 637 -> 372.  Error
-// against 64 bits (2-norm, K 2048 / 5632 / 16384): 7.0e-7 / 1.21e-6 / 2.23e-6,
-// fp32 products 8.1e-7 / 1.34e-6 / 2.29e-6.
+// MI355X, against fp32 products on the skinny kernel: 300 x 11264 x 2048 158 ->
+// 109 us, 300 x 2048 x 5632 85 -> 56, 512 x 32000 x 2048 616 -> 365.  Parts that
+// are cut off instead of rounded saved 3% and adding products straight into the
+// sum 4% more, but then what is left out or lost has the sign of the product
+// (error x10 on positive data of K 16384).
+// Error against 64 bits (2-norm, K 256 / 2048 / 16384): N(0, 1) 0.7e-7 / 1.6e-7 /
+// 4.3e-7, fp32 products 2.9e-7 / 8.2e-7 / 2.3e-6; uniform in [0, 1) 0.5e-7 /
+// 1.1e-7 / 3.0e-7 against 2.2e-7 / 6.0e-7 / 1.7e-6; all low bits of every
+// operand set 0.5e-7 / 2.2e-7 / 4.2e-7 against 0.5e-7 / 9.7e-6 / 2.9e-5.
 #include "tv_split.h"
 #include "tv_dense.h"
 #include "tv_linear.h"
