@@ -667,6 +667,39 @@ def test_prefill_f32_positive_sums(d):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("eq,ek,ev", [(0, 0, -118), (0, 0, -130), (-118, 119, 0), (119, -118, 0), (0, 0, 100)])
+def test_prefill_f32_range(d, eq, ek, ev):
+    """Queries, keys and values scaled by powers of two lose no low bits.  A score's error is a
+    few 2^-24 of sum |q k|, about 2 sqrt(d) here, and moves the output by as much; values
+    near 2^-130 are rounded to 2^-149 once more on the way out, 2^-19 of the smallest outputs
+    (0.1 of a value's size)."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    n, hq, hkv = 200, 4, 2
+    q, k, v = (randn(350 + i, n, h, d).cuda() * 2.0 ** e for i, (h, e) in enumerate([(hq, eq), (hkv, ek), (hkv, ev)]))
+    out = flash_prefill_attention(q[None], k[None], v[None])[0].double().cpu().numpy()
+    want = attend_visible(q, k, v, True)
+    err = np.linalg.norm(out - want) / np.linalg.norm(want)
+    assert err < 4 * d ** 0.5 * 2.0 ** -24 + (2.0 ** -18 if ev == -130 else 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [2, 300])          # one, two key groups
+def test_prefill_f32_scores_that_overflow_on_the_way(d, n):
+    """The products of a score pass -2^80 before they come back to +2^80: the last key takes all
+    the weight, whatever the partial sums did."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    q, k = torch.zeros(n, 2, d), torch.zeros(n, 1, d)
+    q[:] = 2.0 ** 40
+    k[n - 1, 0, :d // 4] = -1.3 * 2.0 ** 35 * 128 / d
+    k[n - 1, 0, d // 4:] = 0.9 * 2.0 ** 35 * 128 / d
+    v = randn(360, n, 1, d)
+    out = flash_prefill_attention(q.cuda()[None], k.cuda()[None], v.cuda()[None], False)[0].cpu()
+    assert torch.equal(out, v[n - 1].expand(n, 2, d))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
 def test_prefill_f32_non_finite_values(d):
     """Infinities, NaN and values near the fp32 limit reach the rows that see them and no other."""
     from tinyvllm_amd.attention import flash_prefill_attention

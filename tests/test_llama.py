@@ -244,6 +244,23 @@ def test_linear_f32_many_rows_parts(low_bits, terms):
     assert ((out.double() - want).abs() <= 2.5 * 2.0 ** -24 * want.abs()).all()
 
 
+@pytest.mark.parametrize("ea,ew", [(-118, 60), (60, -118), (-130, 90), (-149, 100), (70, -3), (110, -100)])
+def test_linear_f32_many_rows_range(ea, ew):
+    """Operands of 2^ea and 2^ew: small ones lose no low bits (a part below the smallest bf16
+    number would be 1e-5 of the result and more), large ones are multiplied in fp32.  256
+    products: a walk of at most sqrt(256) 2^-24 of the sum's own size, as for N(0, 1)."""
+    from tinyvllm_amd._lib import TV_F32
+    M, N, K = 70, 132, 256
+    a = gen(46, M, K, dtype=torch.float32) * 2.0 ** ea if ea > -149 else \
+        torch.randint(-9, 10, (M, K), dtype=torch.float64).mul(2.0 ** -149).float().cuda()
+    w = gen(47, N, K, dtype=torch.float32) * 2.0 ** ew
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, N, K, 2, None, TV_F32, None), "logits")
+    torch.cuda.synchronize()
+    want = a.double() @ w.double().T.contiguous()
+    assert ((out.double() - want).norm() / want.norm()).item() < 16 * 2.0 ** -24
+
+
 def test_linear_f32_many_rows_non_finite():
     """Infinities, NaN and values beyond the largest bf16 give what fp32 products give."""
     from tinyvllm_amd._lib import TV_F32

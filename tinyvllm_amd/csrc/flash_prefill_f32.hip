@@ -18,8 +18,8 @@
 // The split costs about as many issue slots per tile as the products, so
 // neither unit is full; two work-groups (or key groups) per CU overlap them.
 // MI355X, causal, against one wave per query row on the VALU: Hq 32 / Hkv 4,
-// head_dim 64: L 64 8.9 -> 6.0 us, L 512 174 -> 18, L 1500 1347 -> 71; Hkv 8,
-// head_dim 128: L 512 354 -> 31, L 1500 2834 -> 150 (123 TFLOP/s of attention).
+// head_dim 64: L 64 8.9 -> 6.5 us, L 512 174 -> 19, L 1500 1347 -> 75; Hkv 8,
+// head_dim 128: L 512 354 -> 33, L 1500 2834 -> 157 (118 TFLOP/s of attention).
 // Error against 64 bits (2-norm; L 64 / 300 / 700): N(0, 1) 0.8e-7 / 1.1e-7 /
 // 1.1e-7, the VALU kernel 1.8e-7 / 3.1e-7 / 3.0e-7; scores of standard deviation
 // 6: 1.9e-7 / 2.8e-7 / 3.0e-7 against 4.7e-7 / 9.8e-7 / 8.3e-7.
@@ -47,7 +47,7 @@ template <bool PAGED> __device__ __forceinline__ long long key_row(const Prefill
 
 // One query row by one wave in plain fp32 arithmetic, each key's value touched
 // only where the key is visible: the rows whose result above is not finite
-// (infinities or NaN among the inputs, or values near the fp32 limit).
+// (infinities or NaN among the inputs, or values beyond tv_split.h's range).
 template <int D, bool PAGED>
 __device__ __forceinline__ void exact_row(const PrefillParams& p, int h, int qi, float* sp) {
   const int lane = threadIdx.x & 63;
@@ -214,6 +214,7 @@ prefill_f32_kernel(const PrefillParams p) {
 #pragma unroll
   for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   float mref = 0.0f, thr = -__FLT_MAX__, lsum = 0.0f;   // rescale threshold: -FLT_MAX until the first visible key
+  float lowest = 0.0f;                                  // smallest score, before scale and mask
 
   auto compute = [&](int t) {
     const int k0 = t * kBN;
@@ -229,10 +230,15 @@ prefill_f32_kernel(const PrefillParams p) {
           kf[q] = *reinterpret_cast<const u32x4*>(tile + q * PLANE + (kb * 16 + col) * KP + ks * 32 + g * 8);
         s[kb] += mfma_split(kf, qf[ks], f32x4{0.f, 0.f, 0.f, 0.f});
       }
+    // a score of -inf is one whose sum overflowed on its way (the inputs have no
+    // infinities, or it would be NaN): its row is repeated in plain fp32
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      lowest = fminf(lowest, fminf(fminf(s[kb][0], s[kb][1]), fminf(s[kb][2], s[kb][3])));
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[kb][i] = fmaf(s[kb][i], c, -mref);
+      for (int i = 0; i < 4; ++i) s[kb][i] = fmaf(s[kb][i] * kSplitUnscale, c, -mref);
     if (!(k0 + kBN <= p.kv_len && (!p.causal || k0 + kBN - 1 <= row0 + qoff))) {
       const int rel = (p.causal ? min(p.kv_len - 1, qi + qoff) : p.kv_len - 1) - (k0 + 4 * g);   // last visible key
 #pragma unroll
@@ -287,7 +293,7 @@ prefill_f32_kernel(const PrefillParams p) {
     if (grp + KS * j < ntiles) compute(grp + KS * j);
   }
 
-  float l = sum_over_g(lsum);
+  float l = sum_over_g(lowest > kNegInf ? lsum : __builtin_nanf(""));
   if constexpr (KS > 1) {
     float* so = reinterpret_cast<float*>(smem);   // [KS][64 rows][MP]
     float* ssum = so + KS * kBM * MP;             // [KS][64 rows]
@@ -319,7 +325,7 @@ prefill_f32_kernel(const PrefillParams p) {
     }
   }
 
-  const float inv = bad ? __builtin_nanf("") : 1.0f / l;
+  const float inv = bad ? __builtin_nanf("") : kSplitUnscale / l;
   bool finite = true;
 #pragma unroll
   for (int db = 0; db < DB; ++db) {

@@ -10,13 +10,13 @@
 // so fragment reads and writes touch every bank once.
 //
 // What bounds it: the matrix unit at the rate it sustains (512 x 32000 x 2048:
-// 365 us, 1.10 PFLOP/s of bf16; the 16-bit product reaches 1.23), and below
-// that size the split, which takes its issue slots (64 x 128 tile: 528 clocks
+// 375 us, 1.07 PFLOP/s of bf16; the 16-bit product reaches 1.23), and below
+// that size the split, which takes its issue slots (64 x 128 tile: 620 clocks
 // of a stage beside 768 of products).  Four work-groups per CU of the smaller
 // tile (118 registers) run their splits beside each other's products; two with
 // a second stage buffer, split and products interleaved, were 3% slower.
 // MI355X, against fp32 products on the skinny kernel: 300 x 11264 x 2048 158 ->
-// 109 us, 300 x 2048 x 5632 85 -> 56, 512 x 32000 x 2048 616 -> 365.  Parts that
+// 117 us, 300 x 2048 x 5632 122 -> 58, 512 x 32000 x 2048 616 -> 375.  Parts that
 // are cut off instead of rounded saved 3% and adding products straight into the
 // sum 4% more, but then what is left out or lost has the sign of the product
 // (error x10 on positive data of K 16384).
@@ -173,15 +173,17 @@ tile_linear_f32_kernel(const LinearParams p) {
     }
   }
 
-  // Infinities, NaN or values near the fp32 limit do not split: a wave with a
-  // result that is not finite recomputes its part from fp32 products.
+  // Infinities, NaN, operands of 2^104 and results of 2^80 do not split: a wave
+  // with a result that is not finite recomputes its part from fp32 products.
   bool finite = true;
 #pragma unroll
   for (int mb = 0; mb < MBW; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[mb][nb][i]) < __builtin_inff();
+      acc[mb][nb] *= kSplitUnscale;
+    }
   if (__builtin_amdgcn_ballot_w64(!finite) != 0) {
 #pragma unroll
     for (int mb = 0; mb < MBW; ++mb)

@@ -21,7 +21,20 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& 
   m = pack2<__bf16>(a, b);
   l = __builtin_amdgcn_perm(bits(b - bf16_hi(m)), bits(a - bf16_lo(m)), 0x07060302u);   // upper halves: the rest is zero
 }
+
+// Operands are scaled by 2^24 before they are split: the lowest bit of the
+// smallest fp32 number (2^-149) is then a normal bf16 number, so the sum of the
+// parts is exact for every operand and not only above 2^-110, whatever the
+// matrix core does with subnormals.  Operands of 2^104 and more overflow, and so
+// do sums of 2^80 and more; the caller sees both as results that are not finite
+// and repeats them in plain fp32.
+constexpr float kSplitScale = 0x1p24f;
+constexpr float kSplitUnscale = 0x1p-48f;   // of a product of two
+
+// Split eight operands.
 __device__ __forceinline__ void split8(f32x4 a, f32x4 b, u32x4 (&s)[3]) {
+  a *= kSplitScale;
+  b *= kSplitScale;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     uint32_t h, m, l;
@@ -33,7 +46,7 @@ __device__ __forceinline__ void split8(f32x4 a, f32x4 b, u32x4 (&s)[3]) {
 }
 __device__ __forceinline__ f32x4 as_f32x4(u32x4 w) { return __builtin_bit_cast(f32x4, w); }
 
-// c += A B from the parts of both, smallest products first.  The three products
+// c += 2^48 A B from the parts of both, smallest products first.  The three products
 // of the lowest parts are left out: at most 0.992 * 2^-24 of the whole product
 // (the largest over all 2^23 significands, m = 1 - 2^-8 half steps), zero on
 // average.
