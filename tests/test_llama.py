@@ -282,6 +282,34 @@ def test_linear_f32_many_rows_non_finite():
     assert (np.abs(got - want)[ok] <= 2e-5 * mag[ok]).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,K,ks", [(33, 64, 64), (64, 96, 96), (20, 1056, 352), (40, 2816, 2816), (64, 1280, 1280)])
+def test_linear_non_finite_weights(dtype, M, K, ks):
+    """An infinity or NaN in W reaches its own feature's sum and no other: not that of the row
+    before (K ends inside a chunk), of the split before, nor, as NaN, its own through the
+    chunks that pad an odd count."""
+    from tinyvllm_amd._lib import dtype_code
+    N = 68
+    a = gen(48, M, K, dtype=dtype).abs() + 0.5
+    w = gen(49, N, K, dtype=dtype, scale=0.05)
+    w[3, 0], w[20, K - 1], w[41, ks // 2] = float("inf"), float("-inf"), float("nan")
+    splits = -(-K // ks)
+    out = torch.empty((splits, M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, 0, ks, 0, None, dtype_code(dtype), None), "partial")
+    torch.cuda.synchronize()
+    for s in range(splits):
+        k = slice(s * ks, (s + 1) * ks)
+        finite = np.nan_to_num(f64(w)[:, k], nan=0, posinf=0, neginf=0).T
+        want, mag = f64(a)[:, k] @ finite, f64(a)[:, k] @ np.abs(finite)
+        for row, col, x in ((3, 0, np.inf), (20, K - 1, -np.inf), (41, ks // 2, np.nan)):
+            if s * ks <= col < (s + 1) * ks:
+                want[:, row] = x
+        got = out[s].double().cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        ok = np.isfinite(want)
+        assert (np.abs(got[ok] - want[ok]) <= 2e-5 * mag[ok]).all()
+
+
 def test_greedy_tie_resolves_to_first_index():
     """Two identical, dominant rows in different work-group tiles (5 and 70): every
     token ties between them and must take 5 (numpy / tinygrad argmax semantics)."""

@@ -95,7 +95,10 @@ __device__ __forceinline__ void linear_epilogue(const LinearParams& p, const f32
   }
 }
 
-template <typename T, int EPI>
+// TAIL: K ranges that end inside a chunk.  What lies past them in W's rows (other
+// splits, the next row) is then not read: a product with a zero of A would make
+// NaN of an infinity or NaN there.
+template <typename T, int EPI, bool TAIL>
 __global__ void __launch_bounds__(256, kLinearMinBlocks) linear_kernel(const LinearParams p) {
   // LDS in 16-bit units; a chunk row is 512 bytes of K at a 544-byte pitch (an
   // odd multiple of 32 modulo 256: conflict-free 16-byte reads)
@@ -128,23 +131,25 @@ __global__ void __launch_bounds__(256, kLinearMinBlocks) linear_kernel(const Lin
   // return zero in hardware, so no address is clamped.  The row part of every
   // offset goes in the VGPR offset: the hardware range check covers the VGPR
   // and instruction offsets, not the scalar one.
-  const long long w_rows = max(p.N - n_wave, 0);
+  // (16 rows of W, so that offsets from 2^31 on are past its range)
+  const unsigned w_rows = __builtin_amdgcn_readfirstlane(min(max(p.N - n_wave, 0), 16));
   const __amdgpu_buffer_rsrc_t wres = make_rsrc(reinterpret_cast<const T*>(p.w) + (size_t)min(n_wave, p.N) * p.K,
-                                                (unsigned long long)w_rows * p.K * sizeof(T));
+                                                (unsigned long long)w_rows * (unsigned)p.K * sizeof(T));
   const __amdgpu_buffer_rsrc_t ares = make_rsrc(reinterpret_cast<const T*>(p.a) + (size_t)m0 * p.lda,
                                                 (unsigned long long)max(p.M - m0, 0) * p.lda * sizeof(T));
   const int w_voff = (col * p.K + kb) * (int)sizeof(T) + 16 * g;
   const int a_voff = ((tid >> 5) * (int)p.lda + kb) * (int)sizeof(T) + 16 * (tid & 31);
   const int a_rows8 = 8 * (int)p.lda * (int)sizeof(T);   // byte step between the 8 rows a thread loads
 
-  // W: lane (row col, k group g) reads 16 bytes per 64-byte k step.  Columns
-  // past the split are multiplied by zero rows of A.
+  // W: lane (row col, k group g) reads 16 bytes per 64-byte k step.
   // i is the position in this work-group's chunk sequence; positions past the
-  // last chunk re-read it (W) or load zeros (A), so padding steps add nothing.
+  // last chunk load zeros, so padding steps add nothing.
   auto loadW = [&](int i, u32x4 (&r)[8]) {
-    const int off = w_voff + chunk_of(min(i, nc - 1)) * 512;
+    const int c = chunk_of(min(i, nc - 1));
+    const int off = i < nc ? w_voff + c * 512 : (int)0x80000000;
+    const int left = (ke - kb) * (int)sizeof(T) - c * 512;   // bytes of a row from this chunk on
 #pragma unroll
-    for (int s = 0; s < 8; ++s) r[s] = buffer_load16(wres, off + 64 * s, 0);
+    for (int s = 0; s < 8; ++s) r[s] = buffer_load16(wres, !TAIL || 64 * s < left ? off + 64 * s : (int)0x80000000, 0);
   };
   // A chunk: 64 rows x 32 vectors of 16 bytes; thread tid loads vector
   // tid % 32 of rows tid / 32 + 8 i.  Columns past the split are zeroed when
@@ -389,6 +394,15 @@ template <typename T, int EPI> static void launch_few(const LinearParams& p, hip
   else hipLaunchKernelGGL((few_linear_kernel<T, EPI, KW, 16, 2>), grid, dim3(256), 0, s, p);
 }
 
+template <typename T, int EPI> static void launch_skinny(const LinearParams& p, hipStream_t s) {
+  const dim3 grid((p.K + p.k_split - 1) / p.k_split, (p.N + kLinBN - 1) / kLinBN, (p.M + kLinBM - 1) / kLinBM);
+  constexpr int KC = 512 / (int)sizeof(T);
+  if (p.K % KC || (p.k_split < p.K && p.k_split % KC))
+    hipLaunchKernelGGL((linear_kernel<T, EPI, true>), grid, dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL((linear_kernel<T, EPI, false>), grid, dim3(256), 0, s, p);
+}
+
 template <typename T> static void launch_linear_t(const LinearParams& p, int epi, hipStream_t s) {
   constexpr long long ES = sizeof(T);
   if (p.M <= kFewRows && std::max<long long>(p.lda, p.K) * ES * 16 < (1LL << 31)) {   // 32-bit offsets in 16 rows
@@ -397,10 +411,9 @@ template <typename T> static void launch_linear_t(const LinearParams& p, int epi
     else launch_few<T, kEpiLogits>(p, s);
     return;
   }
-  const dim3 grid((p.K + p.k_split - 1) / p.k_split, (p.N + kLinBN - 1) / kLinBN, (p.M + kLinBM - 1) / kLinBM);
-  if (epi == kEpiPartial) hipLaunchKernelGGL((linear_kernel<T, kEpiPartial>), grid, dim3(256), 0, s, p);
-  else if (epi == kEpiSwiglu) hipLaunchKernelGGL((linear_kernel<T, kEpiSwiglu>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((linear_kernel<T, kEpiLogits>), grid, dim3(256), 0, s, p);
+  if (epi == kEpiPartial) launch_skinny<T, kEpiPartial>(p, s);
+  else if (epi == kEpiSwiglu) launch_skinny<T, kEpiSwiglu>(p, s);
+  else launch_skinny<T, kEpiLogits>(p, s);
 }
 
 void launch_linear(const LinearParams& p, int epi, int dtype, hipStream_t s) {
