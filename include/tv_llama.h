@@ -42,6 +42,15 @@ extern "C" {
  */
 int tv_linear_k_split(int M, int N, int K);
 
+/* The kernel that tv_linear takes for packed rows of A (lda = K). */
+#define TV_LINEAR_SKINNY 0    /* 64 x 64 tiles, W streamed once per 64 rows */
+#define TV_LINEAR_FEW 1       /* at most 16 rows */
+#define TV_LINEAR_TILED_256 2 /* LDS-tiled, 256 x 256 (16-bit types only) */
+#define TV_LINEAR_TILED_128 3 /* 128 x 128 */
+#define TV_LINEAR_TILED_64 4  /* 64 x 128 */
+/* Host-only; -1: bad arguments. */
+int tv_linear_kernel(int M, int N, int K, int k_split, int epilogue, int dtype);
+
 /*
  * Y = A W^T, A [M, K] (row stride lda elements), W [N, K] dense, both of dtype.
  * Replaces tinygrad Linear(bias=False) calls (llama.py:150-153, 214-216, 254).

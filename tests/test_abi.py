@@ -129,6 +129,24 @@ def test_linear_split_choice():
     assert lib.tv_linear_k_split(4, 96, 64) % 32 == 0
 
 
+@pytest.mark.parametrize("dtype,M,N,K,splits,epilogue,tiled", [
+    # measured faster on 64 x 64 tiles: little work for many rows
+    ("F32", 65, 512, 512, 8, 0, False), ("F32", 128, 1024, 1024, 6, 0, False), ("F32", 65, 512, 4096, 16, 0, False),
+    ("F32", 65, 1024, 4096, 1, 1, False), ("F32", 256, 1000, 2048, 1, 2, False), ("F32", 128, 5632, 1024, 1, 1, False),
+    ("F32", 320, 512, 512, 4, 0, False), ("F16", 65, 1024, 1024, 6, 0, False), ("F16", 128, 512, 4096, 16, 0, False),
+    ("BF16", 256, 4096, 256, 1, 0, False), ("BF16", 65, 2816, 1024, 1, 1, False), ("F16", 320, 1024, 4096, 1, 1, False),
+    ("F16", 128, 1000, 2048, 1, 2, False),
+    # and on the tiled kernels
+    ("F32", 300, 11264, 2048, 1, 1, True), ("F32", 512, 32000, 2048, 1, 2, True), ("F32", 300, 2048, 5632, 8, 0, True),
+    ("F16", 1000, 2560, 2048, 1, 0, True), ("BF16", 2048, 32768, 4096, 1, 1, True), ("F16", 300, 2048, 5632, 4, 0, True),
+    ("F16", 128, 11264, 2048, 1, 1, True), ("BF16", 128, 32000, 2048, 1, 2, True)])
+def test_kernel_of_a_many_row_product(dtype, M, N, K, splits, epilogue, tiled):
+    """More than 64 rows go to the tiled kernels only where those are the faster ones."""
+    ks = -(-K // splits // 32) * 32
+    kernel = _lib.load().tv_linear_kernel(M, N, K, ks, epilogue, getattr(_lib, "TV_" + dtype))
+    assert kernel >= 2 if tiled else kernel == 0
+
+
 def test_dense_entry_points_validate_on_host():
     lib = _lib.load()
     p = ctypes.c_void_p(256)

@@ -196,14 +196,18 @@ def test_linear_f32_many_rows(M, N, K, ks):
     check_products(torch.float32, M, N, K, ks)
 
 
-@pytest.mark.parametrize("M,N", [(70, 260), (512, 8260)])       # 64 x 128, 128 x 128 tiles
-def test_linear_f32_many_rows_positive_sums(M, N):
+TILED_128, TILED_64 = 3, 4     # tv_linear_kernel: 128 x 128 and 64 x 128 tiles
+
+
+@pytest.mark.parametrize("M,N,kernel", [(65, 20484, TILED_128), (193, 6148, TILED_64)])
+def test_linear_f32_many_rows_positive_sums(M, N, kernel):
     """Sums of 16384 positive products: 512 stages, each rounded into the sum by 2^-24 of it at
     most and without a bias, so the error walks to about sqrt(512) 2^-24 = 1.3e-6 of the sum.
     (Low parts added to the whole sum one by one are lost once it is 2^8 products long, always
     with the same sign: 1.8e-5.)"""
     from tinyvllm_amd._lib import TV_F32
     K = 16384
+    assert lib().tv_linear_kernel(M, N, K, K, 2, TV_F32) == kernel
     g = torch.Generator().manual_seed(44)
     a, w = (torch.rand((n, K), generator=g).cuda() for n in (M, N))
     out = torch.empty((M, N), dtype=torch.float32, device="cuda")
@@ -215,14 +219,16 @@ def test_linear_f32_many_rows_positive_sums(M, N):
 
 @pytest.mark.parametrize("low_bits", [False, True])
 @pytest.mark.parametrize("terms", [1, 32])
-def test_linear_f32_many_rows_parts(low_bits, terms):
+@pytest.mark.parametrize("M,N,kernel", [(65, 16388, TILED_128), (65, 8196, TILED_64)])
+def test_linear_f32_many_rows_parts(M, N, kernel, low_bits, terms):
     """Every part product counts, and none is one-sided: outputs of one product each, and sums
     of 32 products of one sign, with random significands or with all low bits set.  The products
     left out are at most 2^-24 of the whole; six products are added smallest first, so one
     rounding of 2^-24 and parts of 2^-8 of it follow.  A lost part product is 2^-17 or more,
     parts that are cut off leave 8 * 2^-24."""
     from tinyvllm_amd._lib import TV_F32
-    M, N, K = 96, 260, 32
+    K = 32
+    assert lib().tv_linear_kernel(M, N, K, K, 2, TV_F32) == kernel
     rng = np.random.default_rng(45)
 
     def draw(*shape):
@@ -245,12 +251,14 @@ def test_linear_f32_many_rows_parts(low_bits, terms):
 
 
 @pytest.mark.parametrize("ea,ew", [(-118, 60), (60, -118), (-130, 90), (-149, 100), (70, -3), (110, -100)])
-def test_linear_f32_many_rows_range(ea, ew):
+@pytest.mark.parametrize("M,N,kernel", [(65, 24580, TILED_128), (129, 16388, TILED_64)])
+def test_linear_f32_many_rows_range(M, N, kernel, ea, ew):
     """Operands of 2^ea and 2^ew: small ones lose no low bits (a part below the smallest bf16
     number would be 1e-5 of the result and more), large ones are multiplied in fp32.  256
     products: a walk of at most sqrt(256) 2^-24 of the sum's own size, as for N(0, 1)."""
     from tinyvllm_amd._lib import TV_F32
-    M, N, K = 70, 132, 256
+    K = 256
+    assert lib().tv_linear_kernel(M, N, K, K, 2, TV_F32) == kernel
     a = gen(46, M, K, dtype=torch.float32) * 2.0 ** ea if ea > -149 else \
         torch.randint(-9, 10, (M, K), dtype=torch.float64).mul(2.0 ** -149).float().cuda()
     w = gen(47, N, K, dtype=torch.float32) * 2.0 ** ew

@@ -38,6 +38,7 @@ SIGNATURES = {
     "tv_read_kv_blocks": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P]),
     # include/tv_llama.h
     "tv_linear_k_split": (_I, [_I, _I, _I]),
+    "tv_linear_kernel": (_I, [_I, _I, _I, _I, _I, _I]),
     "tv_linear": (_I, [_P, _P, _P, _I, _I, _I, _L, _L, _I, _I, _P, _I, _P]),
     "tv_rms_norm_residual": (_I, [_P, _P, _P, _I, _P, _P, _I, _P, _I, _I, _F, _I, _P]),
     "tv_rope_table": (_I, [_P, _I, _I, _F, _P]),

@@ -7,10 +7,10 @@
 //   SwiGLU           w2(silu(w1 x) * w3 x)                       llama.py:220-221
 //   greedy sampling  argmax over the vocabulary (first maximum)  sampling.py:131-134
 //
-// linear_kernel computes Y = A W^T for a skinny A (the decode batch, M <= 64
-// per work-group; at most 16 rows: few_linear_kernel; more than 64:
-// tile_linear.hip, tile_linear_f32.hip) against a weight matrix W [N, K] that is streamed from HBM
-// exactly once.  Each of the 4 waves of a work-group owns 16 rows of W and all
+// linear_kernel computes Y = A W^T for a skinny A (the decode batch, 64 rows per
+// work-group; at most 16 rows: few_linear_kernel; more than 64: mostly
+// tile_linear.hip, tile_linear_f32.hip) against a weight matrix W [N, K] that is
+// streamed from HBM once per 64 rows.  Each of the 4 waves of a work-group owns 16 rows of W and all
 // 64 rows of A; A is staged in LDS per 512-byte-wide K chunk (256 fp16/bf16 or
 // 128 fp32 elements) and shared by the waves.  fp32 runs the same byte layout
 // on v_mfma_f32_16x16x4_f32, four of them per 16-byte fragment pair.  W rows are the MFMA A operand (lane = output feature), A^T the B
@@ -403,9 +403,8 @@ template <typename T, int EPI> static void launch_skinny(const LinearParams& p, 
     hipLaunchKernelGGL((linear_kernel<T, EPI, false>), grid, dim3(256), 0, s, p);
 }
 
-template <typename T> static void launch_linear_t(const LinearParams& p, int epi, hipStream_t s) {
-  constexpr long long ES = sizeof(T);
-  if (p.M <= kFewRows && std::max<long long>(p.lda, p.K) * ES * 16 < (1LL << 31)) {   // 32-bit offsets in 16 rows
+template <typename T> static void launch_linear_t(const LinearParams& p, int epi, LinearKernel k, hipStream_t s) {
+  if (k == kLinearFew) {
     if (epi == kEpiPartial) launch_few<T, kEpiPartial>(p, s);
     else if (epi == kEpiSwiglu) launch_few<T, kEpiSwiglu>(p, s);
     else launch_few<T, kEpiLogits>(p, s);
@@ -416,12 +415,107 @@ template <typename T> static void launch_linear_t(const LinearParams& p, int epi
   else launch_skinny<T, kEpiLogits>(p, s);
 }
 
+// K elements per split of a product of at most kFewRows rows (few_linear_kernel):
+// the cheapest of 1 .. 8 splits, in the stages that the busiest work-group
+// walks (its units, each the stages of one wave times four and about three more
+// to start and sum; two more per split for the partials).  MI355X, 4 rows,
+// 1 / 2 / 3 / 4 splits: 2048 x 5632 fp32 14.4 / 12.5 / 13.4 / 12.1 us (takes 2),
+// fp16 8.8 / 7.3 / 7.9 / 7.6 (2); 2560 x 2048 fp16 5.1 / 5.4 / 5.6 / 5.7 (1);
+// 1024 x 2816 fp32 9.0 / 6.7 / 6.1 / 5.9 (3).
+static int few_k_split(int N, int K, int es) {
+  const int nc = (K * es + kFewStage - 1) / kFewStage;
+  const long long tiles = (N + 15) / 16;
+  long long best = 0;
+  int chunks = nc;
+  for (int s = 1; s <= 8 && s <= nc; ++s) {
+    const int per = (nc + s - 1) / s;
+    const long long rounds = (tiles * s + kFewWorkGroups - 1) / kFewWorkGroups;
+    const long long cost = rounds * ((per + 3) / 4 * 4 + 3) + 2 * (s - 1);
+    if (s == 1 || cost < best) {
+      best = cost;
+      chunks = per;
+    }
+  }
+  return (int)std::min<long long>(((long long)K + 31) / 32 * 32, (long long)chunks * (kFewStage / es));
+}
+
+// Work-groups a skinny product aims for when it splits K.
+constexpr long long kLinearTargetWorkGroups = 192;
+
+// K elements per split of linear_kernel for a product whose consumer sums the
+// partials.
+static int skinny_k_split(int M, int N, int K) {
+  const long long full = ((long long)K + 31) / 32 * 32;
+  const long long tiles = ((N + kLinBN - 1) / kLinBN) * (long long)((M + kLinBM - 1) / kLinBM);
+  // About three work-groups per four CUs: more splits add partials that the
+  // consumer (norm or step attention) reads back, and on the TinyLlama step
+  // 192 beat 128, 160, 224 and 256 (1.53 vs 1.55-1.59 ms).
+  const long long target = kLinearTargetWorkGroups;
+  if (tiles >= target / 2) return (int)full;
+  const long long want = (target + tiles - 1) / tiles;
+  const long long per = (K + want - 1) / want;
+  // whole LDS chunks: a partial chunk still streams the chunk's full width of W
+  const long long ks = per >= kLinKC ? (per + kLinKC / 2) / kLinKC * kLinKC : (per + 31) / 32 * 32;
+  return (int)std::min(full, std::max(ks, 32LL));
+}
+
+// Microseconds of linear_kernel: a start, and per round of work-groups the
+// chunks of one (an odd count beyond two runs one more); logits of many rows
+// also wait for their scattered stores.  fp32 is bound by its products, so two
+// work-groups that share a CU take half a round each.  MI355X, M 65 .. 2048, N
+// 512 .. 32768, K 256 .. 16384: most within 15% of the measured time.
+static double skinny_us(int M, int N, int K, int k_split, int dtype, bool logits) {
+  const int kc = dtype == kF32 ? kLinKC / 2 : kLinKC;
+  int chunks = (std::min(k_split, K) + kc - 1) / kc;
+  if (chunks > 2) chunks += chunks & 1;
+  const long long wgs = (long long)((M + kLinBM - 1) / kLinBM) * ((N + kLinBN - 1) / kLinBN) * ((K + k_split - 1) / k_split);
+  const double stores = logits ? 0.6e-6 * M * N : 0.0;
+  if (dtype == kF32) return 2.8 + 2.65 * chunks * std::max(1.0, 0.5 * (double)((wgs + 127) / 128)) + stores;
+  return (chunks == 1 ? 2.7 : 3.5) + 1.35 * chunks * (double)((wgs + 255) / 256) + stores;
+}
+
+// What the consumer of `splits` partials pays for them (about 4 TB/s and a
+// quarter of a microsecond each).
+static double partials_us(int M, int N, int splits) { return (splits - 1) * ((double)M * N * 1e-6 + 0.25); }
+
+// More than kLinBM rows: the LDS-tiled kernels where their model is the smaller
+// one.  They win with many rows, long K or many tiles; where W is small,
+// linear_kernel's 64 x 64 tiles and finer splits fill more of the chip.
+// MI355X, us, linear_kernel / tiled: 65 rows, fp16 1024 x 1024 4.2 / 5.5, 2048 x
+// 2048 9.0 / 7.4; fp32 512 x 512 5.4 / 13.9, 1024 x 4096 (SwiGLU) 86 / 170, 2560 x
+// 2048 20.7 / 20.6; 320 rows, fp16 1024 x 512 4.4 / 5.5, 2560 x 2048 16.9 / 12.7;
+// fp32 1024 x 1024 13.7 / 14.9, 11264 x 2048 158 / 117.
+static double tiled_us(int M, int N, int K, int k_split, int dtype) {
+  const int splits = (K + k_split - 1) / k_split;
+  return dtype == kF32 ? tile_linear_f32_us(M, N, K, splits) : tile_linear_us(M, N, K, splits);
+}
+
+int linear_k_split(int M, int N, int K, int dtype) {
+  if (M <= kFewRows) return few_k_split(N, K, dtype == kF32 ? 4 : 2);
+  const int skinny = skinny_k_split(M, N, K);
+  if (M <= kLinBM) return skinny;
+  const int tiled = dtype == kF32 ? tile_linear_f32_k_split(M, N, K) : tile_linear_k_split(M, N, K);
+  const double s = skinny_us(M, N, K, skinny, dtype, false) + partials_us(M, N, (K + skinny - 1) / skinny);
+  const double t = tiled_us(M, N, K, tiled, dtype) + partials_us(M, N, (K + tiled - 1) / tiled);
+  return s < t ? skinny : tiled;
+}
+
+LinearKernel linear_kernel_of(const LinearParams& p, int epi, int dtype) {
+  const long long row = std::max<long long>(p.lda, p.K) * (dtype == kF32 ? 4 : 2);
+  if (p.M <= kFewRows) return row * 16 < (1LL << 31) ? kLinearFew : kLinearSkinny;   // 32-bit offsets in 16 rows
+  if (p.M > kLinBM && (dtype == kF32 ? tile_linear_f32_supported(p) : tile_linear_supported(p)) &&
+      tiled_us(p.M, p.N, p.K, p.k_split, dtype) <= skinny_us(p.M, p.N, p.K, p.k_split, dtype, epi == kEpiLogits))
+    return kLinearTiled;
+  return kLinearSkinny;
+}
+
 void launch_linear(const LinearParams& p, int epi, int dtype, hipStream_t s) {
-  if (tile_linear_supported(p, dtype)) return launch_tile_linear(p, epi, dtype, s);
-  if (dtype == kF32 && tile_linear_f32_supported(p)) return launch_tile_linear_f32(p, epi, s);
-  if (dtype == kF16) launch_linear_t<_Float16>(p, epi, s);
-  else if (dtype == kBF16) launch_linear_t<__bf16>(p, epi, s);
-  else launch_linear_t<float>(p, epi, s);
+  const LinearKernel k = linear_kernel_of(p, epi, dtype);
+  if (k == kLinearTiled && dtype == kF32) launch_tile_linear_f32(p, epi, s);
+  else if (k == kLinearTiled) launch_tile_linear(p, epi, dtype, s);
+  else if (dtype == kF16) launch_linear_t<_Float16>(p, epi, k, s);
+  else if (dtype == kBF16) launch_linear_t<__bf16>(p, epi, k, s);
+  else launch_linear_t<float>(p, epi, k, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -38,51 +38,6 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 int splits_of(int K, int k_split) { return (K + k_split - 1) / k_split; }
 
-// Work-groups a skinny product aims for when it splits K.
-constexpr long long kLinearTargetWorkGroups = 192;
-
-// K elements per split of a product of at most kFewRows rows (few_linear_kernel):
-// the cheapest of 1 .. 8 splits, in the stages that the busiest work-group
-// walks (its units, each the stages of one wave times four and about three more
-// to start and sum; two more per split for the partials).  MI355X, 4 rows,
-// 1 / 2 / 3 / 4 splits: 2048 x 5632 fp32 14.4 / 12.5 / 13.4 / 12.1 us (takes 2),
-// fp16 8.8 / 7.3 / 7.9 / 7.6 (2); 2560 x 2048 fp16 5.1 / 5.4 / 5.6 / 5.7 (1);
-// 1024 x 2816 fp32 9.0 / 6.7 / 6.1 / 5.9 (3).
-int few_k_split(int N, int K, int es) {
-  const int nc = (K * es + tv::kFewStage - 1) / tv::kFewStage;
-  const long long tiles = (N + 15) / 16;
-  long long best = 0;
-  int chunks = nc;
-  for (int s = 1; s <= 8 && s <= nc; ++s) {
-    const int per = (nc + s - 1) / s;
-    const long long rounds = (tiles * s + tv::kFewWorkGroups - 1) / tv::kFewWorkGroups;
-    const long long cost = rounds * ((per + 3) / 4 * 4 + 3) + 2 * (s - 1);
-    if (s == 1 || cost < best) {
-      best = cost;
-      chunks = per;
-    }
-  }
-  return (int)std::min<long long>(round_up(K, 32), (long long)chunks * (tv::kFewStage / es));
-}
-
-// K elements per split of a product whose consumer sums the partials.
-int k_split_of(int M, int N, int K, int dtype) {
-  if (M > tv::kLinBM) return dtype == TV_F32 ? tv::tile_linear_f32_k_split(M, N, K) : tv::tile_linear_k_split(M, N, K);
-  if (M <= tv::kFewRows) return few_k_split(N, K, (int)elem_bytes(dtype));
-  const long long full = round_up(K, 32);
-  const long long tiles = ((N + tv::kLinBN - 1) / tv::kLinBN) * (long long)((M + tv::kLinBM - 1) / tv::kLinBM);
-  // About three work-groups per four CUs: more splits add partials that the
-  // consumer (norm or step attention) reads back, and on the TinyLlama step
-  // 192 beat 128, 160, 224 and 256 (1.53 vs 1.55-1.59 ms).
-  const long long target = kLinearTargetWorkGroups;
-  if (tiles >= target / 2) return (int)full;
-  const long long want = (target + tiles - 1) / tiles;
-  const long long per = (K + want - 1) / want;
-  // whole LDS chunks: a partial chunk still streams the chunk's full width of W
-  const long long ks = per >= tv::kLinKC ? (per + tv::kLinKC / 2) / tv::kLinKC * tv::kLinKC : round_up(per, 32);
-  return (int)std::min(full, std::max(ks, 32LL));
-}
-
 // Carves 256-byte aligned regions out of one workspace.
 struct Carver {
   size_t off = 0;
@@ -126,9 +81,9 @@ StepLayout step_layout(const tv_llama_model* m, int B, int max_blocks, int block
   const int qd = m->n_heads * m->head_dim;
   const int kd = m->n_kv_heads * m->head_dim;
   const int nqkv = qkv_width(m);
-  L.ks_qkv = k_split_of(B, nqkv, m->dim, m->dtype);
-  L.ks_o = k_split_of(B, m->dim, qd, m->dtype);
-  L.ks_2 = k_split_of(B, m->dim, m->hidden_dim, m->dtype);
+  L.ks_qkv = tv::linear_k_split(B, nqkv, m->dim, m->dtype);
+  L.ks_o = tv::linear_k_split(B, m->dim, qd, m->dtype);
+  L.ks_2 = tv::linear_k_split(B, m->dim, m->hidden_dim, m->dtype);
   const size_t part_floats = std::max({(size_t)splits_of(m->dim, L.ks_qkv) * nqkv, (size_t)splits_of(qd, L.ks_o) * m->dim,
                                        (size_t)splits_of(m->hidden_dim, L.ks_2) * m->dim}) * (size_t)B;
   const size_t es = elem_bytes(m->dtype);
@@ -404,7 +359,22 @@ extern "C" {
 
 int tv_linear_k_split(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 32;
-  return k_split_of(M, N, K, TV_F16);
+  return tv::linear_k_split(M, N, K, TV_F16);
+}
+
+int tv_linear_kernel(int M, int N, int K, int k_split, int epilogue, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || k_split <= 0 || !step_dtype(dtype)) return -1;
+  tv::LinearParams p{};
+  p.M = M;
+  p.N = N;
+  p.K = K;
+  p.lda = K;
+  p.k_split = k_split;
+  const int k = tv::linear_kernel_of(p, epilogue, dtype);
+  if (k != tv::kLinearTiled) return k;
+  const int splits = splits_of(K, k_split);
+  return k + (dtype == TV_F32 ? 1 + tv::tile_linear_f32_shape(M, N, K, splits, nullptr)
+                              : tv::tile_linear_shape(M, N, K, splits, nullptr));
 }
 
 int tv_linear(void* out, const void* a, const void* w, int M, int N, int K, int64_t lda, int64_t ldo, int k_split,

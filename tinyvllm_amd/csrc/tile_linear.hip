@@ -239,7 +239,7 @@ static double tile_cost(const TileShape& s, int M, int N, int K, int splits) {
   return stages * std::max(s.alone, s.shared * per_cu);
 }
 
-static int tile_shape(int M, int N, int K, int splits, double* cost = nullptr) {
+int tile_linear_shape(int M, int N, int K, int splits, double* cost) {
   int best = 0;
   double bc = 0.0;
   for (int i = 0; i < 3; ++i) {
@@ -250,6 +250,13 @@ static int tile_shape(int M, int N, int K, int splits, double* cost = nullptr) {
   return best;
 }
 
+// The same with what lies around the stages (most within 15% of the measured time, M 65 .. 2048).
+double tile_linear_us(int M, int N, int K, int splits) {
+  double c;
+  tile_linear_shape(M, N, K, splits, &c);
+  return 2.4 + 1.2 * c;
+}
+
 // Splits of K for a product whose consumer sums partials: the cheapest of 1, 2,
 // 4 and 8 with at least four stages each, charged with the fp32 partials that
 // the consumer reads back (about 4 TB/s) and half a microsecond per doubling.
@@ -258,7 +265,7 @@ int tile_linear_k_split(int M, int N, int K) {
   int ks = (K + 31) / 32 * 32;
   for (int splits = 1; splits <= 8 && (splits == 1 || K / splits >= 256); splits *= 2) {
     double c;
-    tile_shape(M, N, K, splits, &c);
+    tile_linear_shape(M, N, K, splits, &c);
     c += (splits - 1) * ((double)M * N * 1e-6 + 0.25);
     if (splits == 1 || c < best) {
       best = c;
@@ -268,12 +275,9 @@ int tile_linear_k_split(int M, int N, int K) {
   return ks;
 }
 
-// Beyond 64 rows the skinny kernel streams W once per 64 tokens, at a quarter
-// of the LDS-tiled rate (M 65, 2048 x 2048: 8.3 against 6.1 us; M 1000,
-// 11264 x 2048: 125 against 53 us); at 64 and below it is the faster one (M 64,
-// 2048 x 5632: 9.3 against 10.0 us).  32-bit offsets inside a tile.
-bool tile_linear_supported(const LinearParams& p, int dtype) {
-  return dtype != kF32 && p.M > kLinBM && std::max<long long>(p.lda, p.K) * 2 * 256 < (1LL << 31);
+// 32-bit offsets inside a tile.
+bool tile_linear_supported(const LinearParams& p) {
+  return std::max<long long>(p.lda, p.K) * 2 * 256 < (1LL << 31);
 }
 
 template <typename T, int MBW, int WM, int WN, int S>
@@ -293,7 +297,7 @@ static void launch_tile(const LinearParams& p, int epi, int splits, hipStream_t 
 
 template <typename T> static void launch_tile_t(const LinearParams& p, int epi, hipStream_t s) {
   const int splits = (p.K + p.k_split - 1) / p.k_split;
-  switch (tile_shape(p.M, p.N, p.K, splits)) {
+  switch (tile_linear_shape(p.M, p.N, p.K, splits, nullptr)) {
     case 0: launch_tile<T, 8, 2, 4, 2>(p, epi, splits, s); break;   // 256 x 256, 128 KB of LDS, one per CU
     case 1: launch_tile<T, 4, 2, 2, 2>(p, epi, splits, s); break;   // 128 x 128, 64 KB, two per CU
     default: launch_tile<T, 2, 2, 2, 3>(p, epi, splits, s);         // 64 x 128, 72 KB, two per CU

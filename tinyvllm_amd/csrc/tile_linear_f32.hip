@@ -223,11 +223,18 @@ static double tile_cost_f32(const TileShapeF32& s, int M, int N, int K, int spli
   return stages * std::max(s.alone, s.start + s.each * per_cu);
 }
 
-static int tile_shape_f32(int M, int N, int K, int splits, double* cost = nullptr) {
+int tile_linear_f32_shape(int M, int N, int K, int splits, double* cost) {
   const double a = tile_cost_f32(kTileShapesF32[0], M, N, K, splits);
   const double b = tile_cost_f32(kTileShapesF32[1], M, N, K, splits);
   if (cost) *cost = std::min(a, b);
   return b < a ? 1 : 0;
+}
+
+// The same with what lies around the stages (within 15% of the measured time, M 65 .. 512).
+double tile_linear_f32_us(int M, int N, int K, int splits) {
+  double c;
+  tile_linear_f32_shape(M, N, K, splits, &c);
+  return 2.1 + 1.15 * c;
 }
 
 int tile_linear_f32_k_split(int M, int N, int K) {
@@ -235,7 +242,7 @@ int tile_linear_f32_k_split(int M, int N, int K) {
   int ks = (K + 31) / 32 * 32;
   for (int splits = 1; splits <= 8 && (splits == 1 || K / splits >= 256); splits *= 2) {
     double c;
-    tile_shape_f32(M, N, K, splits, &c);
+    tile_linear_f32_shape(M, N, K, splits, &c);
     c += (splits - 1) * ((double)M * N * 1e-6 + 0.25);   // the partials, read back by the consumer
     if (splits == 1 || c < best) {
       best = c;
@@ -246,7 +253,7 @@ int tile_linear_f32_k_split(int M, int N, int K) {
 }
 
 bool tile_linear_f32_supported(const LinearParams& p) {
-  return p.M > kLinBM && std::max<long long>(p.lda, p.K) * 4 * 128 < (1LL << 31);   // 32-bit offsets in a tile
+  return std::max<long long>(p.lda, p.K) * 4 * 128 < (1LL << 31);   // 32-bit offsets in a tile
 }
 
 template <int MBW, int WM, int WN, int WPE>
@@ -260,7 +267,7 @@ static void launch_tile_f32(const LinearParams& p, int epi, int splits, hipStrea
 
 void launch_tile_linear_f32(const LinearParams& p, int epi, hipStream_t s) {
   const int splits = (p.K + p.k_split - 1) / p.k_split;
-  if (tile_shape_f32(p.M, p.N, p.K, splits) == 0) launch_tile_f32<4, 2, 2, 2>(p, epi, splits, s);   // 48 KB of LDS, two per CU
+  if (tile_linear_f32_shape(p.M, p.N, p.K, splits, nullptr) == 0) launch_tile_f32<4, 2, 2, 2>(p, epi, splits, s);   // 48 KB of LDS, two per CU
   else launch_tile_f32<2, 2, 2, 4>(p, epi, splits, s);                                             // 36 KB, four
 }
 

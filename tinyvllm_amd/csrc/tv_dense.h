@@ -99,13 +99,22 @@ bool step_attn_supported(int head_dim, int group, int block_size);
 void launch_step_attn(const StepAttnParams& p, int head_dim, int dtype, hipStream_t s);
 
 void launch_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
-// many-row products (tile_linear.hip)
-bool tile_linear_supported(const LinearParams& p, int dtype);
+int linear_k_split(int M, int N, int K, int dtype);   // of a product whose consumer sums the partials
+// The kernel that launch_linear takes: linear_kernel, few_linear_kernel, or the
+// tiled ones.
+enum LinearKernel : int { kLinearSkinny = 0, kLinearFew = 1, kLinearTiled = 2 };
+LinearKernel linear_kernel_of(const LinearParams& p, int epilogue, int dtype);
+// many-row products (tile_linear.hip, tile_linear_f32.hip): limits, tile shape, splits of K, estimated time
+bool tile_linear_supported(const LinearParams& p);
+int tile_linear_shape(int M, int N, int K, int splits, double* cost);
 int tile_linear_k_split(int M, int N, int K);
-bool tile_linear_f32_supported(const LinearParams& p);   // tile_linear_f32.hip
-int tile_linear_f32_k_split(int M, int N, int K);
-void launch_tile_linear_f32(const LinearParams& p, int epilogue, hipStream_t s);
+double tile_linear_us(int M, int N, int K, int splits);
 void launch_tile_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
+bool tile_linear_f32_supported(const LinearParams& p);
+int tile_linear_f32_shape(int M, int N, int K, int splits, double* cost);
+int tile_linear_f32_k_split(int M, int N, int K);
+double tile_linear_f32_us(int M, int N, int K, int splits);
+void launch_tile_linear_f32(const LinearParams& p, int epilogue, hipStream_t s);
 void launch_norm(const NormParams& p, int dtype, hipStream_t s);
 void launch_qkv_rope(const QKVParams& p, int dtype, hipStream_t s);
 void launch_rope_table(float* table, int max_pos, int head_dim, float theta, hipStream_t s);
