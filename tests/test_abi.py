@@ -147,6 +147,20 @@ def test_kernel_of_a_many_row_product(dtype, M, N, K, splits, epilogue, tiled):
     assert kernel >= 2 if tiled else kernel == 0
 
 
+@pytest.mark.parametrize("dtype,M,N,K,epilogue,few", [
+    # measured faster on 64 x 64 tiles: one or two chunks of K under many features
+    ("F16", 4, 32768, 256, 1, False), ("F16", 16, 32768, 512, 1, False), ("BF16", 4, 8192, 256, 1, False),
+    ("F16", 16, 16384, 384, 1, False), ("F16", 4, 16384, 256, 0, False), ("F32", 4, 32768, 128, 1, False),
+    ("F32", 16, 16384, 128, 0, False), ("F16", 16, 32000, 256, 2, False),
+    # and on the kernel that streams W past few rows
+    ("F16", 4, 11264, 2048, 1, True), ("BF16", 16, 5632, 512, 1, True), ("F16", 16, 32768, 768, 1, True),
+    ("F16", 1, 32000, 2048, 2, True), ("F32", 16, 11264, 2048, 1, True), ("F32", 4, 8192, 256, 1, True),
+    ("F32", 16, 32000, 128, 2, True), ("F16", 16, 6144, 2048, 0, True)])
+def test_kernel_of_a_few_row_product(dtype, M, N, K, epilogue, few):
+    kernel = _lib.load().tv_linear_kernel(M, N, K, K, epilogue, getattr(_lib, "TV_" + dtype))
+    assert kernel == (1 if few else 0)
+
+
 def test_dense_entry_points_validate_on_host():
     lib = _lib.load()
     p = ctypes.c_void_p(256)

@@ -256,8 +256,10 @@ __global__ void __launch_bounds__(256, kLinearMinBlocks) linear_kernel(const Lin
 // logits, whose argmax keys cover 64 features).  One work-group per CU walks
 // the units; its loads run ahead across them.  The 64-row kernel spent its
 // time on products for rows that are not there (fp32) and on one 64-row tile
-// per work-group, 176 of them on 256 CUs.  W is read once and non-temporally
-// (32000 x 2048 fp32 48.4 us without, 43.7 with).  MI355X, 4 rows, against the
+// per work-group, 176 of them on 256 CUs.  W is read once and non-temporally:
+// from HBM 3-8% faster (32000 x 2048 fp32 48.4 -> 43.7 us; fp16, 4 rows, 2560 x
+// 2048 5.5 -> 5.1, 2048 x 5632 7.1 -> 6.6); weights that all stay in the 256 MB
+// last-level cache (models of a few layers) lose 2-5% at 4 rows, up to 20% at 16.  MI355X, 4 rows, against the
 // 64-row kernel: 11264 x 2048 fp32 47 -> 19.0 us (4.9 TB/s), 32000 x 2048 87 ->
 // 43.7 (6.0), 2048 x 5632 26 -> 11.5; fp16 15.9 -> 10.8, 31.4 -> 22.7, 9.4 ->
 // 7.0.  At 16 rows, fp16: 16.4 -> 12.7, 31.7 -> 24.5, 9.9 -> 8.1.  Rejected: A
@@ -415,25 +417,28 @@ template <typename T> static void launch_linear_t(const LinearParams& p, int epi
   else launch_skinny<T, kEpiLogits>(p, s);
 }
 
-// K elements per split of a product of at most kFewRows rows (few_linear_kernel):
-// the cheapest of 1 .. 8 splits, in the stages that the busiest work-group
-// walks (its units, each the stages of one wave times four and about three more
-// to start and sum; two more per split for the partials).  MI355X, 4 rows,
-// 1 / 2 / 3 / 4 splits: 2048 x 5632 fp32 14.4 / 12.5 / 13.4 / 12.1 us (takes 2),
-// fp16 8.8 / 7.3 / 7.9 / 7.6 (2); 2560 x 2048 fp16 5.1 / 5.4 / 5.6 / 5.7 (1);
-// 1024 x 2816 fp32 9.0 / 6.7 / 6.1 / 5.9 (3).
+// Work of few_linear_kernel in stages: what the busiest work-group walks (its
+// units, each the stages of one wave times four and about three more to start
+// and sum), and two more per split for the partials.
+static int few_stages(int N, int K, int splits, int es) {
+  const int nc = (K * es + kFewStage - 1) / kFewStage;
+  const int per = (nc + splits - 1) / splits;
+  const long long units = (long long)((N + 15) / 16) * splits;
+  return (int)((units + kFewWorkGroups - 1) / kFewWorkGroups) * ((per + 3) / 4 * 4 + 3) + 2 * (splits - 1);
+}
+
+// K elements per split of few_linear_kernel: the cheapest of 1 .. 8 splits.
+// MI355X, 4 rows, 1 / 2 / 3 / 4 splits: 2048 x 5632 fp32 14.4 / 12.5 / 13.4 /
+// 12.1 us (takes 2), fp16 8.8 / 7.3 / 7.9 / 7.6 (2); 2560 x 2048 fp16 5.1 / 5.4 /
+// 5.6 / 5.7 (1); 1024 x 2816 fp32 9.0 / 6.7 / 6.1 / 5.9 (3).
 static int few_k_split(int N, int K, int es) {
   const int nc = (K * es + kFewStage - 1) / kFewStage;
-  const long long tiles = (N + 15) / 16;
-  long long best = 0;
-  int chunks = nc;
+  int best = 0, chunks = nc;
   for (int s = 1; s <= 8 && s <= nc; ++s) {
-    const int per = (nc + s - 1) / s;
-    const long long rounds = (tiles * s + kFewWorkGroups - 1) / kFewWorkGroups;
-    const long long cost = rounds * ((per + 3) / 4 * 4 + 3) + 2 * (s - 1);
+    const int cost = few_stages(N, K, s, es);
     if (s == 1 || cost < best) {
       best = cost;
-      chunks = per;
+      chunks = (nc + s - 1) / s;
     }
   }
   return (int)std::min<long long>(((long long)K + 31) / 32 * 32, (long long)chunks * (kFewStage / es));
@@ -490,19 +495,47 @@ static double tiled_us(int M, int N, int K, int k_split, int dtype) {
   return dtype == kF32 ? tile_linear_f32_us(M, N, K, splits) : tile_linear_us(M, N, K, splits);
 }
 
+// At most kFewRows rows: microseconds of few_linear_kernel, its share of the
+// partials in few_stages.  linear_kernel is the faster one where a work-group
+// has one or two chunks: K up to 512 elements under many features (fp16, 4 rows,
+// SwiGLU: 32768 x 256 6.1 us against 10.7, 8192 x 256 3.9 / 4.9; fp32 32768 x 128
+// 7.6 / 13.3).  Alone it is so too where it splits K that far (fp16, 16 rows:
+// 2048 x 2048 4.1 against 5.0 us, 1024 x 2816 3.8 / 4.6), but into 8 and 11 parts
+// against 2 and 3, which the next kernel reads: steps of eight TinyLlama layers
+// with these products on linear_kernel take 352 us instead of 346 (4 rows), 392
+// instead of 388 (16).
+static double few_us(int M, int N, int K, int k_split, int dtype) {
+  const int stages = few_stages(N, K, (K + k_split - 1) / k_split, dtype == kF32 ? 4 : 2);
+  if (dtype == kF32) return 3.0 + 0.18 * stages;
+  return M <= 4 ? 3.2 + 0.138 * stages : 4.1 + 0.14 * stages;
+}
+
+static bool few_is_faster(int M, int N, int K, int k_split, int dtype, int epi) {
+  // one unit of the logits is 64 features: only a single short chunk is faster
+  // on 64 x 64 tiles
+  if (epi == kEpiLogits) return dtype == kF32 || K > kLinKC || N > 512 * kLinBN;
+  return few_us(M, N, K, k_split, dtype) < skinny_us(M, N, K, k_split, dtype, false);
+}
+
 int linear_k_split(int M, int N, int K, int dtype) {
-  if (M <= kFewRows) return few_k_split(N, K, dtype == kF32 ? 4 : 2);
   const int skinny = skinny_k_split(M, N, K);
+  double s = skinny_us(M, N, K, skinny, dtype, false);
+  if (M <= kFewRows) {
+    const int few = few_k_split(N, K, dtype == kF32 ? 4 : 2);
+    s += partials_us(M, N, (K + skinny - 1) / skinny);
+    return s <= few_us(M, N, K, few, dtype) ? skinny : few;
+  }
   if (M <= kLinBM) return skinny;
   const int tiled = dtype == kF32 ? tile_linear_f32_k_split(M, N, K) : tile_linear_k_split(M, N, K);
-  const double s = skinny_us(M, N, K, skinny, dtype, false) + partials_us(M, N, (K + skinny - 1) / skinny);
+  s += partials_us(M, N, (K + skinny - 1) / skinny);
   const double t = tiled_us(M, N, K, tiled, dtype) + partials_us(M, N, (K + tiled - 1) / tiled);
   return s < t ? skinny : tiled;
 }
 
 LinearKernel linear_kernel_of(const LinearParams& p, int epi, int dtype) {
   const long long row = std::max<long long>(p.lda, p.K) * (dtype == kF32 ? 4 : 2);
-  if (p.M <= kFewRows) return row * 16 < (1LL << 31) ? kLinearFew : kLinearSkinny;   // 32-bit offsets in 16 rows
+  if (p.M <= kFewRows)   // 32-bit offsets in 16 rows
+    return row * 16 < (1LL << 31) && few_is_faster(p.M, p.N, p.K, p.k_split, dtype, epi) ? kLinearFew : kLinearSkinny;
   if (p.M > kLinBM && (dtype == kF32 ? tile_linear_f32_supported(p) : tile_linear_supported(p)) &&
       tiled_us(p.M, p.N, p.K, p.k_split, dtype) <= skinny_us(p.M, p.N, p.K, p.k_split, dtype, epi == kEpiLogits))
     return kLinearTiled;
