@@ -191,7 +191,7 @@ typedef struct tv_llama_prefill_args {
   int attend_prefix;
 } tv_llama_prefill_args;
 
-/* Workspace of tv_llama_prefill.  Host-only. */
+/* Workspace of tv_llama_prefill for up to num_tokens tokens.  Host-only. */
 size_t tv_llama_prefill_workspace_bytes(const tv_llama_model* model, int num_tokens);
 
 /*

@@ -161,6 +161,25 @@ def test_kernel_of_a_few_row_product(dtype, M, N, K, epilogue, few):
     assert kernel == (1 if few else 0)
 
 
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+@pytest.mark.parametrize("dim,heads,kv_heads,hidden", [(2048, 32, 4, 5632), (4096, 32, 8, 16384), (1024, 16, 4, 2816),
+                                                       (512, 8, 2, 1376), (64, 4, 2, 256), (768, 12, 12, 3072)])
+def test_a_prefill_workspace_serves_every_smaller_count(dtype, dim, heads, kv_heads, hidden):
+    """A caller sizes one buffer for its longest prompt.  Shorter ones are split further along K,
+    so they can hold more partials than a long one."""
+    from tinyvllm_amd.llama import _Model
+    lib = _lib.load()
+    m = _Model(n_layers=1, dim=dim, n_heads=heads, n_kv_heads=kv_heads, head_dim=dim // heads, hidden_dim=hidden,
+               vocab_size=32000, dtype=getattr(_lib, "TV_" + dtype))
+    need = [lib.tv_llama_prefill_workspace_bytes(ctypes.byref(m), n) for n in range(1, 2200)]
+    assert all(a <= b for a, b in zip(need, need[1:]))
+    if dtype != "F32":
+        qd, nqkv = dim, dim + 2 * kv_heads * (dim // heads)
+        for n in list(range(1, 70)) + list(range(96, 2200, 37)):
+            for N, K in ((nqkv, dim), (dim, qd), (dim, hidden)):
+                assert -(-K // lib.tv_linear_k_split(n, N, K)) * n * N * 4 <= need[n - 1]
+
+
 def test_dense_entry_points_validate_on_host():
     lib = _lib.load()
     p = ctypes.c_void_p(256)

@@ -75,6 +75,25 @@ int validate_model(const tv_llama_model* m, const char* who) {
 
 int qkv_width(const tv_llama_model* m) { return (m->n_heads + 2 * m->n_kv_heads) * m->head_dim; }
 
+// Rows of partials (splits x M) that a product of up to M rows writes: a
+// workspace of M rows serves every smaller count too, though fewer rows are
+// often split further.  The estimates behind linear_k_split change at rows 5, 17
+// and 65 + 64 j.  Between these, rows only make partials dearer, so beyond 16
+// the first row of a range has the most splits; at most 16 rows have two
+// candidates, and the largest count is that of one end.
+size_t part_rows(int M, int N, int K, int dtype) {
+  size_t rows = 0;
+  for (int first = 1; first <= M;) {
+    const int next = first == 1 ? 5 : first == 5 ? 17 : first == 17 ? 65 : first + 64;
+    const int last = std::min(M, next - 1);
+    int splits = splits_of(K, tv::linear_k_split(first, N, K, dtype));
+    if (first < 17) splits = std::max(splits, splits_of(K, tv::linear_k_split(last, N, K, dtype)));
+    rows = std::max(rows, (size_t)splits * last);
+    first = next;
+  }
+  return rows;
+}
+
 StepLayout step_layout(const tv_llama_model* m, int B, int max_blocks, int block_size, int partition_size,
                        bool decode) {
   StepLayout L{};
@@ -84,8 +103,8 @@ StepLayout step_layout(const tv_llama_model* m, int B, int max_blocks, int block
   L.ks_qkv = tv::linear_k_split(B, nqkv, m->dim, m->dtype);
   L.ks_o = tv::linear_k_split(B, m->dim, qd, m->dtype);
   L.ks_2 = tv::linear_k_split(B, m->dim, m->hidden_dim, m->dtype);
-  const size_t part_floats = std::max({(size_t)splits_of(m->dim, L.ks_qkv) * nqkv, (size_t)splits_of(qd, L.ks_o) * m->dim,
-                                       (size_t)splits_of(m->hidden_dim, L.ks_2) * m->dim}) * (size_t)B;
+  const size_t part_floats = std::max({part_rows(B, nqkv, m->dim, m->dtype) * nqkv, part_rows(B, m->dim, qd, m->dtype) * m->dim,
+                                       part_rows(B, m->dim, m->hidden_dim, m->dtype) * m->dim});
   const size_t es = elem_bytes(m->dtype);
   Carver c;
   L.part = c.take(part_floats * 4);
