@@ -775,3 +775,24 @@ def test_prefill_paged_128_row_kernel_divides_by_the_rounded_weights(dtype):
     w = torch.exp(q[:, :, 0].double() * 16 / d ** 0.5)
     want = v[70].double().repeat_interleave(hq // hkv, 0) * (w / (w + 1))[:, :, None]
     assert ((out - want).abs() <= 1e-4 * want.abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float16, None), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("row", [63, 64, 191, 340, 999])       # first row that sees the invalid block
+def test_prefill_paged_128_row_kernel_invalid_block_in_half_a_tile(dtype, out_dtype, row):
+    """The 64-row query tiles whose keys include an invalid block are NaN; the rows before them
+    are those of a valid table, in the same 128-row tile too, whatever block 0 holds."""
+    from tinyvllm_amd.attention import flash_prefill_paged
+    hq, hkv, d, n, start, bs = 64, 8, 128, 1000, 64, 8
+    nb = (start + n) // bs + 1
+    q, kc, vc = (randn(370 + i, *s, dtype=dtype).cuda()
+                 for i, s in enumerate([(n, hq, d), (nb, bs, hkv, d), (nb, bs, hkv, d)]))
+    table = torch.arange(1, nb, dtype=torch.int32).cuda()       # block 0 is not the sequence's
+    good = flash_prefill_paged(q, kc, vc, table, start, out_dtype=out_dtype)[0]
+    kc[0], vc[0] = float("nan"), float("nan")
+    for bad_id in (nb, -1):
+        table[(start + row) // bs] = bad_id
+        out = flash_prefill_paged(q, kc, vc, table, start, out_dtype=out_dtype)[0]
+        first = row // bs * bs // 64 * 64
+        assert torch.isnan(out[first:]).all() and torch.equal(out[:first], good[:first])

@@ -157,7 +157,7 @@ prefill_rows_kernel(const PrefillParams pa) {
   static_assert(NI >= 1 && NI * 4 * 1024 == TILEB, "tile / DMA shape");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NB * BUFB];
   __shared__ int stbl[PAGED ? kRowsTableMax : 1];
-  __shared__ int sbad;
+  __shared__ int sbad;      // first table entry that is not a block
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -226,7 +226,6 @@ prefill_rows_kernel(const PrefillParams pa) {
   const unsigned long long vstep = (unsigned long long)BN * vstr;
   const int lg = p.kv_bs_log2;
   const int kpad = min(klim, (kend + 2 * BN - 1) / BN * BN);   // end of the keys that are requested
-  bool bad = false;
   int nextid[NI];          // block ids of the next request
   auto request_key = [&](int t, int i) {
     return min(min(t, ntiles - 1) * BN + (wave * NI + i) * RPI, kpad - 1);
@@ -238,9 +237,9 @@ prefill_rows_kernel(const PrefillParams pa) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int key = min(t, ntiles - 1) * BN + (wave * NI + i) * RPI;
-        const int rows = min(RPI, kpad - key);      // keys past the last: zeros
-        const unsigned long long row =
-            ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(nextid[i]) << lg) + (key & ((1 << lg) - 1));
+        const int id = __builtin_amdgcn_readfirstlane(nextid[i]);
+        const int rows = id < 0 ? 0 : min(RPI, kpad - key);   // keys past the last, or in no block: zeros
+        const unsigned long long row = ((unsigned long long)(unsigned)id << lg) + (key & ((1 << lg) - 1));
         rk[i] = rsrc_words(kbase + row * kstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)kstr + ROWB) : 0);
         rv[i] = rsrc_words(vbase + row * vstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)vstr + ROWB) : 0);
       }
@@ -269,14 +268,14 @@ prefill_rows_kernel(const PrefillParams pa) {
   // The Q loads are the only global loads the compiler tracks; retire them
   // here so its own wait for them cannot land inside the tile loop (where it
   // would also drain the LDS-DMA loads in flight).
-  if constexpr (PAGED) {   // an invalid id reads block 0 (in bounds) and makes the rows NaN
-    if (threadIdx.x == 0) sbad = 0;
+  if constexpr (PAGED) {   // keys of an invalid id read as zeros, and the 64-row tiles that see one become NaN
+    if (threadIdx.x == 0) sbad = 0x7FFFFFFF;
     lds_barrier();
     for (int i = threadIdx.x; i <= (kpad - 1) >> lg; i += 256) {
       const int b = p.kv_table[i];
       const bool ok = (unsigned)b < (unsigned)p.kv_num_blocks;
-      stbl[i] = ok ? b : 0;
-      if (!ok && i <= (kend - 1) >> lg) sbad = 1;
+      stbl[i] = ok ? b : -1;
+      if (!ok) atomicMin(&sbad, i);
     }
   }
   wait_vmcnt<0>();
@@ -284,8 +283,10 @@ prefill_rows_kernel(const PrefillParams pa) {
   // zeroed so nothing non-finite can reach a masked product.
   for (int i = threadIdx.x; i < NB * BUFB / 16; i += 256) reinterpret_cast<u32x4*>(smem)[i] = u32x4{0, 0, 0, 0};
   lds_barrier();
+  bool bad = false;
   if constexpr (PAGED) {
-    bad = sbad != 0;
+    const int seen = p.causal ? min(klim, row0 / 64 * 64 + 64 + qoff) : klim;   // keys of this wave's 64-row tile
+    bad = sbad <= (seen - 1) >> lg;
 #pragma unroll
     for (int i = 0; i < NI; ++i) nextid[i] = stbl[request_key(0, i) >> lg];
   }
