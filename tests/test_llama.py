@@ -582,6 +582,28 @@ def test_f32_chunk_of_many_rows(dim, heads, kv_heads, rows):
     assert max_err(got, full[45:]) < LOGIT_TOL["float32"]
 
 
+@pytest.mark.parametrize("dim,heads,kv_heads,n", [(512, 8, 2, 200), (1024, 8, 8, 400)])       # head_dim 64, 128
+@pytest.mark.parametrize("row", [0, 37, 150])
+def test_f32_chunk_with_an_invalid_block(dim, heads, kv_heads, n, row):
+    """A block id outside the cache makes the rows NaN that see it and no others, whatever block
+    0 holds: row i of a chunk attends the blocks of positions 0 .. start + i."""
+    cfg = small_config(dim=dim, n_heads=heads, n_kv_heads=kv_heads, dtype="float32", max_seq_len=512)
+    model, kv, *_ = build(cfg, seed=11, num_blocks=40)
+    start = 43
+    table = torch.randperm(39, generator=torch.Generator().manual_seed(3)).int().cuda() + 1      # without block 0
+    toks = np.random.default_rng(27).integers(0, cfg.vocab_size, start + n)
+    model.prefill_table(toks[:start], kv, table, 0, logits=None)
+    good = model.prefill_table(toks[start:], kv, table, start, attend_prefix=True)[0]
+    at = (start + row) // 16
+    first = max(0, at * 16 - start)               # first row that sees that block
+    for c in kv.k_cache + kv.v_cache:
+        c[0] = float("nan")
+    table[at] = 40
+    out = model.prefill_table(toks[start:], kv, table, start, attend_prefix=True)[0]
+    assert torch.isnan(out[first:]).all()
+    assert not first or max_err(out[:first].cpu().numpy(), good[:first].cpu().numpy()) < LOGIT_TOL["float32"]
+
+
 def prefill_batch(model, kv, bm, ref, rk, rv, lens, rng, cfg):
     """Prefill each sequence on both sides; returns the oracle's next tokens."""
     nxt = []

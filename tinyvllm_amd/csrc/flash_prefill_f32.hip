@@ -108,7 +108,7 @@ prefill_f32_kernel(const PrefillParams p) {
   __shared__ __attribute__((aligned(16))) uint16_t smem[SMEM];
   __shared__ float redo[4][64];
   __shared__ int stbl[PAGED ? kPagedTableMax : 1];
-  __shared__ int sbad;
+  __shared__ int sbad;                    // first table entry that is not a block
 
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
   const int tid = threadIdx.x - grp * GT;
@@ -151,18 +151,18 @@ prefill_f32_kernel(const PrefillParams p) {
   const int lg = p.kv_bs_log2;
   const int kstage = paged_stage_end(0, kend);
   bool bad = false;
-  if constexpr (PAGED) {   // block ids of keys [0, kend); an invalid id reads block 0 and makes the rows NaN
+  if constexpr (PAGED) {   // block ids of keys [0, kend); an invalid id reads block 0, and the rows that see it become NaN
     const int nblk = paged_staged_blocks(0, kstage, lg);
-    if (threadIdx.x == 0) sbad = 0;
+    if (threadIdx.x == 0) sbad = 0x7FFFFFFF;
     lds_barrier();
     for (int i = threadIdx.x; i < nblk; i += blockDim.x) {
       const int b = p.kv_table[i];
       const bool ok = (unsigned)b < (unsigned)p.kv_num_blocks;
       stbl[i] = ok ? b : 0;
-      if (!ok) sbad = 1;
+      if (!ok) atomicMin(&sbad, i);
     }
     lds_barrier();
-    bad = sbad != 0;
+    bad = sbad <= (p.causal ? min(p.kv_len - 1, qi + qoff) : p.kv_len - 1) >> lg;
   }
   struct Stage {
     u32x4 k[NV][2], v[NV][2];
