@@ -652,6 +652,21 @@ def test_prefill_f32_split_products(d, hq, hkv, lq, lk, causal):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,lq,lk,causal", [(8, 12, 12, True), (8, 13, 13, True), (2, 20, 20, True), (2, 21, 21, True),
+                                             (32, 32, 32, True), (32, 33, 33, True), (16, 44, 44, True), (16, 45, 45, True), (4, 64, 64, True),
+                                             (4, 300, 20, True), (4, 20, 300, True), (4, 3, 21, False), (4, 300, 12, False)])
+def test_prefill_f32_few_keys(d, hq, lq, lk, causal):
+    """Both sides of the line between the generic kernel and the one on split products."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    q, k, v = (randn(380 + i, n, h, d).cuda() for i, (n, h) in enumerate([(lq, hq), (lk, hq // 2), (lk, hq // 2)]))
+    out = flash_prefill_attention(q[None], k[None], v[None], causal)[0].double().cpu().numpy()
+    want = attend_visible(q, k, v, causal)
+    # a score errs by a few 2^-24 of sum |q k|, about 2 sqrt(d) here, a weight and the output by as much
+    assert np.linalg.norm(out - want) < 4 * d ** 0.5 * 2.0 ** -24 * np.linalg.norm(want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
 def test_prefill_f32_positive_sums(d):
     """Equal weights over 32768 positive values: the sum of a key group's 512 (or 256) tiles
     walks by at most 2^-24 of it per tile, about sqrt(512) 2^-24 = 1.3e-6 in the end; the row sum
@@ -684,7 +699,7 @@ def test_prefill_f32_range(d, eq, ek, ev):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("n", [2, 300])          # one, two key groups
+@pytest.mark.parametrize("n", [50, 300])         # one, two key groups
 def test_prefill_f32_scores_that_overflow_on_the_way(d, n):
     """The products of a score pass -2^80 before they come back to +2^80: the last key takes all
     the weight, whatever the partial sums did."""

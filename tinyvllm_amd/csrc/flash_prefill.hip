@@ -748,7 +748,7 @@ int launch_flash_prefill(const PrefillParams& p_in, int dtype, void* workspace, 
     }
     return 0;
   }
-  if (prefill_f32_supported(p_in, dtype)) {
+  if (prefill_f32_supported(p_in, dtype) && prefill_f32_faster(p_in)) {
     launch_prefill_f32(p_in, stream);
     return 0;
   }

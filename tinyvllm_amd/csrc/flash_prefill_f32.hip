@@ -356,6 +356,19 @@ bool prefill_f32_supported(const PrefillParams& p, int dtype) {
          (p.q_len + kBM - 1) / kBM <= 65535;
 }
 
+// A first tile of few keys, or a second one, costs more than the generic kernel's
+// one step of 64 keys, whose rows stop at their last key (MI355X, causal, generic
+// / here: Hq 32, head_dim 64: L 8 3.6 / 4.1 us, 20 4.2 / 4.2, 32 4.8 / 4.3, 40 5.2
+// / 5.7, 48 6.0 / 5.8; Hq 8, head_dim 128: L 8 4.9 / 5.3, 16 5.5 / 5.4, 40 7.3 /
+// 7.7, 48 7.8 / 7.8; Hq 32: L 40 8.1 / 7.8; Hq 2, head_dim 64: L 48 5.1 / 5.6).
+bool prefill_f32_faster(const PrefillParams& p) {
+  const int keys = p.causal ? std::min(p.q_len, p.kv_len) : p.kv_len;
+  if (keys <= (p.head_dim == 64 ? 20 : 12)) return false;
+  if (!p.causal || keys <= kBN || keys > 2 * kBN) return true;
+  const int few = p.head_dim == 64 ? (p.num_heads <= 4 ? kBN : 12) : (p.num_heads <= 16 ? 12 : 0);
+  return keys > kBN + few;
+}
+
 template <bool PAGED> static void launch_f32(const PrefillParams& p, int ks, hipStream_t s) {
   const dim3 grid(p.num_heads, (p.q_len + kBM - 1) / kBM);
   if (p.head_dim == 64) {

@@ -225,9 +225,10 @@ bool attend_prefix_f32(const tv_llama_model* m, const tv_llama_cache* c, const L
   // A row block walks the whole prefix whatever rows it has; with few rows and
   // heads the paged decode of each row, which spreads over the CUs, is shorter.
   // MI355X, two layers over 2040 cached tokens, rows paged / here: 32 heads of
-  // 128, 64 rows 1074 / 1144 us, 100 rows 2082 / 2020; 16 heads of 64, 64 rows
-  // 230 / 248, 100 rows 268 / 267; 32 heads of 64, 48 rows 398 / 389.
-  if ((long long)io.M * m->n_heads * 64 < 1536LL * m->head_dim) return false;
+  // 128 (8 of KV) 80 rows 1250 / 1267 us, 112 rows 1340 / 1311; 32 of 64 (4) 48
+  // rows 391 / 390, 80 rows 521 / 495; 16 of 64 (4) 112 rows 272 / 283, 160 rows
+  // 392 / 338; 8 of 64 (2) 256 rows 228 / 238.
+  if ((long long)io.M * m->n_heads * 64 < 1792LL * m->head_dim) return false;
   if ((bs & (bs - 1)) || (kv_len + bs - 1) / bs > tv::kPagedTableMax) return false;
   tv::PrefillParams p{};
   p.out = io.attn;

@@ -99,6 +99,7 @@ int launch_flash_prefill_paged(const PrefillParams& p, int dtype, hipStream_t st
 int launch_flash_prefill_varlen(const PrefillParams& p, int num_seqs, int max_q_len, int max_kv_len,
                                 long long total_q, int dtype, hipStream_t stream);
 bool prefill_f32_supported(const PrefillParams& p, int dtype);
+bool prefill_f32_faster(const PrefillParams& p);   // than the generic kernel (contiguous keys)
 void launch_prefill_f32(const PrefillParams& p, hipStream_t stream);   // contiguous or paged (kv_table set) keys
 void launch_kv_write(const KVWriteParams& p, int vec_bytes, hipStream_t stream);
 void launch_kv_gather(const KVGatherParams& p, int vec_bytes, hipStream_t stream);
