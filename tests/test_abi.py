@@ -161,6 +161,24 @@ def test_kernel_of_a_few_row_product(dtype, M, N, K, epilogue, few):
     assert kernel == (1 if few else 0)
 
 
+@pytest.mark.parametrize("dtype,es", [("F32", 4), ("F16", 2), ("BF16", 2)])
+def test_products_of_rows_beyond_32_bit_offsets_are_refused(dtype, es):
+    """16 rows of W and 64 of A have to lie within 4 GiB, or 16 of both within 2 GiB for at most 16
+    rows (nothing is launched)."""
+    lib, p = _lib.load(), 0x1000
+    code = getattr(_lib, "TV_" + dtype)
+
+    def refused(M, K, lda):
+        rc = lib.tv_linear(p, p, p, M, 64, K, lda, 0, K, 0, None, code, None)
+        return rc == _lib.TV_EUNSUPPORTED and b"32-bit" in lib.tv_last_error()
+
+    assert refused(4, (1 << 32) // (16 * es) + 32, (1 << 32) // (16 * es) + 32)
+    for M in (2, 4, 16):
+        assert refused(M, 64, (1 << 31) // (16 * es))
+    for M in (17, 64, 65, 1000):
+        assert refused(M, 64, (1 << 32) // (64 * es) + 8)
+
+
 @pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
 @pytest.mark.parametrize("dim,heads,kv_heads,hidden", [(2048, 32, 4, 5632), (4096, 32, 8, 16384), (1024, 16, 4, 2816),
                                                        (512, 8, 2, 1376), (64, 4, 2, 256), (768, 12, 12, 3072)])

@@ -290,6 +290,24 @@ def test_linear_f32_many_rows_non_finite():
     assert (np.abs(got - want)[ok] <= 2e-5 * mag[ok]).all()
 
 
+@pytest.mark.parametrize("M,es_lda", [(1, 1 << 33), (4, (1 << 27) - 32), (17, 1 << 26), (70, 1 << 26)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_linear_rows_far_apart(dtype, M, es_lda):
+    """The longest strides of A that are taken: rows 2^26 (2^27: at most 16 rows) bytes apart."""
+    from tinyvllm_amd._lib import dtype_code
+    N, K, lda = 68, 64, es_lda // dtype.itemsize
+    buf = torch.empty((M - 1) * lda + K, dtype=dtype, device="cuda")
+    rows = gen(50, M, K, dtype=dtype)
+    for m in range(M):
+        buf[m * lda:m * lda + K] = rows[m]
+    w = gen(51, N, K, dtype=dtype, scale=0.05)
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(buf), ptr(w), M, N, K, lda, 0, K, 0, None, dtype_code(dtype), None), "partial")
+    torch.cuda.synchronize()
+    want, mag = f64(rows) @ f64(w).T, np.abs(f64(rows)) @ np.abs(f64(w)).T
+    assert (np.abs(f64(out) - want) <= 2e-6 * mag).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,K,ks", [(33, 64, 64), (64, 96, 96), (20, 1056, 352), (40, 2816, 2816), (64, 1280, 1280)])
 def test_linear_non_finite_weights(dtype, M, K, ks):

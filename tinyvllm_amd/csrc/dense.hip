@@ -532,10 +532,27 @@ int linear_k_split(int M, int N, int K, int dtype) {
   return s < t ? skinny : tiled;
 }
 
+// 32-bit offsets: in the 16 rows that few_linear_kernel addresses, and in the 16
+// rows of W and 64 of A (those past M too, which a wrapped offset would bring back
+// into range) of linear_kernel.
+static bool few_supported(int M, int K, long long lda, int dtype) {
+  return M <= kFewRows && std::max<long long>(lda, K) * (dtype == kF32 ? 4 : 2) * 16 < (1LL << 31);
+}
+static bool skinny_supported(int K, long long lda, int dtype) {
+  const long long es = dtype == kF32 ? 4 : 2;
+  return K * es * 16 <= (1LL << 32) && lda <= (1LL << 32) / (es * kLinBM);
+}
+// The tiled kernels' limits lie within linear_kernel's.
+bool linear_supported(int M, int K, long long lda, int dtype) {
+  return few_supported(M, K, lda, dtype) || skinny_supported(K, lda, dtype);
+}
+
 LinearKernel linear_kernel_of(const LinearParams& p, int epi, int dtype) {
-  const long long row = std::max<long long>(p.lda, p.K) * (dtype == kF32 ? 4 : 2);
-  if (p.M <= kFewRows)   // 32-bit offsets in 16 rows
-    return row * 16 < (1LL << 31) && few_is_faster(p.M, p.N, p.K, p.k_split, dtype, epi) ? kLinearFew : kLinearSkinny;
+  if (p.M <= kFewRows) {
+    if (!few_supported(p.M, p.K, p.lda, dtype)) return kLinearSkinny;
+    return !skinny_supported(p.K, p.lda, dtype) || few_is_faster(p.M, p.N, p.K, p.k_split, dtype, epi) ? kLinearFew
+                                                                                                      : kLinearSkinny;
+  }
   if (p.M > kLinBM && (dtype == kF32 ? tile_linear_f32_supported(p) : tile_linear_supported(p)) &&
       tiled_us(p.M, p.N, p.K, p.k_split, dtype) <= skinny_us(p.M, p.N, p.K, p.k_split, dtype, epi == kEpiLogits))
     return kLinearTiled;

@@ -73,6 +73,15 @@ int validate_model(const tv_llama_model* m, const char* who) {
   return TV_OK;
 }
 
+// The products of M rows over the widths that have no limit of their own.
+int validate_widths(const tv_llama_model* m, int M, const char* who) {
+  const long long qd = (long long)m->n_heads * m->head_dim;
+  if (qd > 0x7fffffff || !tv::linear_supported(M, (int)qd, qd, m->dtype) ||
+      !tv::linear_supported(M, m->hidden_dim, m->hidden_dim, m->dtype))
+    return fail(TV_EUNSUPPORTED, "%s: rows of %lld or %d elements are too long for 32-bit offsets", who, qd, m->hidden_dim);
+  return TV_OK;
+}
+
 int qkv_width(const tv_llama_model* m) { return (m->n_heads + 2 * m->n_kv_heads) * m->head_dim; }
 
 // Rows of partials (splits x M) that a product of up to M rows writes: a
@@ -414,7 +423,9 @@ int tv_linear(void* out, const void* a, const void* w, int M, int N, int K, int6
   if (epilogue == TV_EPI_LOGITS && out && (ldo < N || ldo % 4 || !aligned16(out)))
     return fail(TV_EINVAL, "tv_linear: logits output needs ldo >= N, ldo %% 4 == 0, 16-byte alignment");
   if (epilogue == TV_EPI_PARTIAL && !aligned16(out)) return fail(TV_EINVAL, "tv_linear: partials must be 16-byte aligned");
-  const long long splits = splits_of(K, k_split);
+  if (M == 1) lda = K;   // nothing lies at the stride
+  if (!tv::linear_supported(M, K, lda, dtype))
+    return fail(TV_EUNSUPPORTED, "tv_linear: rows too long for 32-bit offsets (K=%d, lda=%lld)", K, (long long)lda);
   if ((N + tv::kLinBN - 1) / tv::kLinBN > 65535 || (M + tv::kLinBM - 1) / tv::kLinBM > 65535)
     return fail(TV_EINVAL, "tv_linear: grid too large");
   linear(a, w, M, N, K, lda, k_split, epilogue, out, ldo, reinterpret_cast<unsigned long long*>(keys), dtype,
@@ -522,6 +533,7 @@ int tv_llama_decode_step(const tv_llama_model* m, const tv_llama_cache* c, const
       a->bt_stride <= 0 || a->max_blocks <= 0 || a->max_blocks > a->bt_stride || a->partition_size <= 0)
     return fail(TV_EINVAL, "tv_llama_decode_step: bad decode arguments");
   if (a->history && a->history_len <= 0) return fail(TV_EINVAL, "tv_llama_decode_step: bad history_len");
+  if ((rc = validate_widths(m, a->batch, "tv_llama_decode_step")) != TV_OK) return rc;
   if (a->logits && !aligned16(a->logits)) return fail(TV_EINVAL, "tv_llama_decode_step: logits must be 16-byte aligned");
   const StepLayout L = step_layout(m, a->batch, a->max_blocks, c->block_size, a->partition_size, true);
   if (!a->workspace || a->workspace_bytes < L.total || !aligned16(a->workspace))
@@ -622,6 +634,7 @@ int tv_llama_prefill(const tv_llama_model* m, const tv_llama_cache* c, const tv_
     return fail(TV_EINVAL, "tv_llama_prefill: bad prefill arguments");
   if (a->logits && !aligned16(a->logits)) return fail(TV_EINVAL, "tv_llama_prefill: logits must be 16-byte aligned");
   const int M = a->num_tokens;
+  if ((rc = validate_widths(m, M, "tv_llama_prefill")) != TV_OK) return rc;
   if ((long long)a->start_pos + M > (long long)a->bt_width * c->block_size)
     return fail(TV_EINVAL, "tv_llama_prefill: the block table covers %lld positions, the chunk ends at %lld",
                 (long long)a->bt_width * c->block_size, (long long)a->start_pos + M);

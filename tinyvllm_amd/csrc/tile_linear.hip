@@ -275,9 +275,10 @@ int tile_linear_k_split(int M, int N, int K) {
   return ks;
 }
 
-// 32-bit offsets inside a tile.
+// 32-bit offsets inside a tile, and threads of the grid.
 bool tile_linear_supported(const LinearParams& p) {
-  return std::max<long long>(p.lda, p.K) * 2 * 256 < (1LL << 31);
+  const long long tiles = (long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * ((p.K + p.k_split - 1) / p.k_split);
+  return std::max<long long>(p.lda, p.K) * 2 * 256 < (1LL << 31) && tiles <= 1 << 23;
 }
 
 template <typename T, int MBW, int WM, int WN, int S>

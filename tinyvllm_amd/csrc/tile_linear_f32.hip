@@ -253,7 +253,9 @@ int tile_linear_f32_k_split(int M, int N, int K) {
 }
 
 bool tile_linear_f32_supported(const LinearParams& p) {
-  return std::max<long long>(p.lda, p.K) * 4 * 128 < (1LL << 31);   // 32-bit offsets in a tile
+  // 32-bit offsets inside a tile, and threads of the grid
+  const long long tiles = (long long)((p.M + 63) / 64) * ((p.N + 127) / 128) * ((p.K + p.k_split - 1) / p.k_split);
+  return std::max<long long>(p.lda, p.K) * 4 * 128 < (1LL << 31) && tiles <= 1 << 23;
 }
 
 template <int MBW, int WM, int WN, int WPE>

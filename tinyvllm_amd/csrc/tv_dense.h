@@ -15,7 +15,7 @@ constexpr int kFewWorkGroups = 256;  // its work-groups: one per CU
 constexpr int kFewStage = 512;       // bytes of a row of W per stage of a wave
 constexpr int kLinKC = 256;   // K elements per LDS chunk at 16-bit types (512 bytes; 128 at fp32)
 
-// Y = A W^T over the K range of one split; grid (splits, ceil(N/64), ceil(M/64)).
+// Y = A W^T over the K range of one split.
 struct LinearParams {
   const void* a;          // [M, K] at row stride lda
   const void* w;          // [N, K] dense
@@ -99,6 +99,7 @@ bool step_attn_supported(int head_dim, int group, int block_size);
 void launch_step_attn(const StepAttnParams& p, int head_dim, int dtype, hipStream_t s);
 
 void launch_linear(const LinearParams& p, int epilogue, int dtype, hipStream_t s);
+bool linear_supported(int M, int K, long long lda, int dtype);
 int linear_k_split(int M, int N, int K, int dtype);   // of a product whose consumer sums the partials
 // The kernel that launch_linear takes: linear_kernel, few_linear_kernel, or the
 // tiled ones.
