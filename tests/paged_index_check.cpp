@@ -12,6 +12,15 @@
 // exits 1.  `planted` replaces the clamp to the staged range by a clamp to the
 // sequence's last key (a former bug) to show the check catches it.
 //
+//   paged_index_check rows q_len start_pos block_size causal [planted]
+//
+// The same for the paged 128-row kernel: for every 128-row query tile, every
+// request of its loop (pairs of 32-key tiles, two pairs ahead, chunks of four
+// rows), checks that the slot lies inside the staged table, that the table fits
+// kRowsTableMax, that the rows read stay below the sequence's end, inside one
+// block and inside the request, and that the tiles' own requests read every key
+// of the unit.  `planted` stages the table to the unit's last key only.
+//
 //   paged_index_check split max_nqt [planted]
 //
 // For every tile count nqt <= max_nqt and first split tile 1 <= split <= nqt
@@ -88,7 +97,53 @@ static int check_split(int max_nqt, bool planted) {
   return 0;
 }
 
+static int check_rows(int q_len, int start, int bs, bool causal, bool planted) {
+  int lg = 0;
+  while ((1 << lg) < bs) ++lg;
+  if ((1 << lg) != bs || bs < tv::kRowsChunk) return 2;
+  const int kv_len = start + q_len, rows = 128, bn = 32;
+  long long checked = 0;
+  for (int qt = 0; qt * rows < q_len; ++qt) {
+    const int kend = tv::prefill_unit_key_end(causal, kv_len, qt, rows, start);
+    const int ntiles = (kend + bn - 1) / bn;
+    const int end = tv::rows_paged_end(kv_len, kend, bn);
+    const int staged = ((planted ? kend : end) - 1 >> lg) + 1;
+    if (staged > tv::kRowsTableMax || staged > (kv_len + bs - 1) / bs) {
+      std::printf("table of %d blocks (unit %d)\n", staged, qt);
+      return 1;
+    }
+    std::vector<char> read(kend, 0);
+    for (int t = 0; t <= ntiles + 4; ++t)
+      for (int row = 0; row < bn; row += tv::kRowsChunk) {
+        const int key = tv::rows_request_key(t, ntiles, bn, row);
+        const int slot = tv::rows_request_slot(key, end, lg);
+        const int n = tv::rows_request_rows(key, end);
+        ++checked;
+        if (slot < 0 || slot >= staged) {
+          std::printf("unit %d tile %d row %d key %d slot %d of %d staged\n", qt, t, row, key, slot, staged);
+          return 1;
+        }
+        if (n <= 0) continue;
+        if (n > tv::kRowsChunk || key + n > kv_len || key >> lg != slot || (key + n - 1) >> lg != slot) {
+          std::printf("unit %d tile %d row %d: keys [%d, %d) of block %d\n", qt, t, row, key, key + n, slot);
+          return 1;
+        }
+        if (t < ntiles)
+          for (int j = key; j < key + n && j < kend; ++j) read[j] = 1;
+      }
+    for (int j = 0; j < kend; ++j)
+      if (!read[j]) {
+        std::printf("unit %d: key %d is not read\n", qt, j);
+        return 1;
+      }
+  }
+  std::printf("ok %lld\n", checked);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc >= 6 && std::strcmp(argv[1], "rows") == 0)
+    return check_rows(std::atoi(argv[2]), std::atoi(argv[3]), std::atoi(argv[4]), std::atoi(argv[5]) != 0, argc > 6);
   if (argc >= 3 && std::strcmp(argv[1], "split") == 0) return check_split(std::atoi(argv[2]), argc > 3);
   if (argc < 5) {
     std::fprintf(stderr, "usage: %s q_len start_pos block_size causal [planted]\n", argv[0]);

@@ -60,6 +60,25 @@ def test_the_old_clamp_reads_past_the_staged_table(checker):
     assert res.returncode == 1 and "slot" in res.stdout, res.stdout + res.stderr
 
 
+ROWS_CASES = [
+    # the 128-row kernel's: the GPU tests' shapes, the measured chunk, the longest table (2048 blocks)
+    (1000, 77, 16, True), (1024, 0, 4, True), (901, 640, 32, True), (1000, 64, 8, True), (2048, 2048, 16, True),
+    (1000, 7192, 4, True), (1000, 31768, 16, True), (1000, 77, 16, False), (1, 0, 4, True), (129, 3, 4, True),
+    (128, 96, 32, True), (2047, 6145, 4, False),
+]
+
+
+@pytest.mark.parametrize("q_len,start,bs,causal", ROWS_CASES)
+def test_every_request_of_the_128_row_kernel_maps_to_a_staged_slot(checker, q_len, start, bs, causal):
+    res = subprocess.run([str(checker), "rows", *map(str, (q_len, start, bs, int(causal)))], capture_output=True, text=True)
+    assert res.returncode == 0 and res.stdout.startswith("ok "), res.stdout + res.stderr
+
+
+def test_a_table_staged_to_the_last_key_only_is_caught(checker):
+    res = subprocess.run([str(checker), "rows", "1000", "77", "16", "1", "planted"], capture_output=True, text=True)
+    assert res.returncode == 1 and "slot" in res.stdout, res.stdout + res.stderr
+
+
 def test_split_units_cover_every_query_tile_once(checker):
     """The 128-row kernel's split grids (tinyvllm_amd/csrc/flash_prefill_rows.hip):
     every tile count up to 64 (L 8192) and every first split tile."""

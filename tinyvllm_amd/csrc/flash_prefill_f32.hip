@@ -19,7 +19,7 @@
 // neither unit is full; two work-groups (or key groups) per CU overlap them.
 // MI355X, causal, against one wave per query row on the VALU: Hq 32 / Hkv 4,
 // head_dim 64: L 64 8.9 -> 6.5 us, L 512 174 -> 19, L 1500 1347 -> 75; Hkv 8,
-// head_dim 128: L 512 354 -> 33, L 1500 2834 -> 157 (118 TFLOP/s of attention).
+// head_dim 128: L 512 354 -> 33, L 1500 2834 -> 148 (125 TFLOP/s of attention).
 // Error against 64 bits (2-norm; L 64 / 300 / 700): N(0, 1) 0.8e-7 / 1.1e-7 /
 // 1.1e-7, the VALU kernel 1.8e-7 / 3.1e-7 / 3.0e-7; scores of standard deviation
 // 6: 1.9e-7 / 2.8e-7 / 3.0e-7 against 4.7e-7 / 9.8e-7 / 8.3e-7.
@@ -386,12 +386,14 @@ void launch_prefill_f32(const PrefillParams& p_in, hipStream_t s) {
   p.xcd_remap = p.num_heads % 8 == 0;
   // Key groups shorten the chain of the longest row (about 1 us per 32 keys):
   // two beyond 64 keys (MI355X, Hq 32 / Hkv 4, head_dim 64, one / two: L 64 5.9 /
-  // 6.2 us, L 300 15.8 / 13.1, L 1024 45.9 / 35.8, L 1500 71.9 / 69.6; head_dim
-  // 128, Hkv 8: L 512 39.0 / 30.2, L 1500 144 / 144); four at head_dim 64 where
-  // the grid leaves CUs with one work-group (L 512 19.3 with two, 18.0; L 300
-  // 13.1, 13.4).
+  // 6.1 us, L 300 17.9 / 13.8, L 1024 51.5 / 37.9, L 1500 77 / 72; head_dim 128,
+  // Hkv 8: L 512 40.2 / 31.9), but not at head_dim 128 where the grid fills every
+  // CU twice (L 1024 77 / 79, L 1500 145 / 153); four at head_dim 64 where it leaves
+  // CUs with one work-group (L 512 20.2 with two, 18.6; L 300 13.8, 13.7).
   const long long wgs = (long long)p.num_heads * ((p.q_len + kBM - 1) / kBM);
-  const int ks = p.kv_len <= 64 ? 1 : (wgs <= 256 && p.kv_len >= 384 ? 4 : 2);
+  int ks = 2;
+  if (p.kv_len <= 64 || (p.head_dim == 128 && wgs >= 512)) ks = 1;
+  else if (wgs <= 256 && p.kv_len >= 384) ks = 4;   // (head_dim 128: two)
   if (p.kv_table) launch_f32<true>(p, ks, s);
   else launch_f32<false>(p, ks, s);
 }

@@ -225,20 +225,19 @@ prefill_rows_kernel(const PrefillParams pa) {
   const unsigned long long kstep = (unsigned long long)BN * kstr;
   const unsigned long long vstep = (unsigned long long)BN * vstr;
   const int lg = p.kv_bs_log2;
-  const int kpad = min(klim, (kend + 2 * BN - 1) / BN * BN);   // end of the keys that are requested
+  const int kpad = rows_paged_end(klim, kend, BN);
   int nextid[NI];          // block ids of the next request
-  auto request_key = [&](int t, int i) {
-    return min(min(t, ntiles - 1) * BN + (wave * NI + i) * RPI, kpad - 1);
-  };
+  static_assert(!PAGED || RPI == kRowsChunk, "one block per request");
+  auto request_key = [&](int t, int i) { return rows_request_key(t, ntiles, BN, (wave * NI + i) * RPI); };
   auto issue = [&](int t) {
     const uint32_t buf = lds0 + (uint32_t)((t % NB) * BUFB);
     if constexpr (PAGED) {
       u32x4 rk[NI], rv[NI];
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        const int key = min(t, ntiles - 1) * BN + (wave * NI + i) * RPI;
+        const int key = request_key(t, i);
         const int id = __builtin_amdgcn_readfirstlane(nextid[i]);
-        const int rows = id < 0 ? 0 : min(RPI, kpad - key);   // keys past the last, or in no block: zeros
+        const int rows = id < 0 ? 0 : rows_request_rows(key, kpad);   // keys past the last, or in no block: zeros
         const unsigned long long row = ((unsigned long long)(unsigned)id << lg) + (key & ((1 << lg) - 1));
         rk[i] = rsrc_words(kbase + row * kstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)kstr + ROWB) : 0);
         rv[i] = rsrc_words(vbase + row * vstr, rows > 0 ? (unsigned long long)((rows - 1) * (uint32_t)vstr + ROWB) : 0);
@@ -248,7 +247,7 @@ prefill_rows_kernel(const PrefillParams pa) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) load_lds16(rv[i], sgpr(buf + (uint32_t)(TILEB + (wave * NI + i) * 1024)), vvoff[i]);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) nextid[i] = stbl[request_key(t + 1, i) >> lg];
+      for (int i = 0; i < NI; ++i) nextid[i] = stbl[rows_request_slot(request_key(t + 1, i), kpad, lg)];
       return;
     }
     if (t > 0 && t < ntiles) {
@@ -288,7 +287,7 @@ prefill_rows_kernel(const PrefillParams pa) {
     const int seen = p.causal ? min(klim, row0 / 64 * 64 + 64 + qoff) : klim;   // keys of this wave's 64-row tile
     bad = sbad <= (seen - 1) >> lg;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) nextid[i] = stbl[request_key(0, i) >> lg];
+    for (int i = 0; i < NI; ++i) nextid[i] = stbl[rows_request_slot(request_key(0, i), kpad, lg)];
   }
   issue(0);
   issue(1);

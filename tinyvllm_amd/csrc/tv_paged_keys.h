@@ -50,6 +50,28 @@ __host__ __device__ inline int prefill_group_tile(int grp, int groups, int j, in
   return t < ntiles - 1 ? t : ntiles - 1;
 }
 
+// The same for the paged 128-row kernel, which stages the table from key 0 and
+// loads kRowsChunk rows of one block per request.  It asks for tiles up to the
+// pair that holds the last key (the second may be past it), and repeats the last
+// one beyond: keys below rows_paged_end are read, requests at or past it are
+// empty and take the last staged key's slot.
+constexpr int kRowsChunk = 4;
+__host__ __device__ inline int rows_paged_end(int klim, int kend, int tile_keys) {
+  const int pad = (kend + 2 * tile_keys - 1) / tile_keys * tile_keys;
+  return klim < pad ? klim : pad;
+}
+// First key of a request: chunk `row` (a multiple of kRowsChunk) of tile `tile`.
+__host__ __device__ inline int rows_request_key(int tile, int ntiles, int tile_keys, int row) {
+  return (tile < ntiles - 1 ? tile : ntiles - 1) * tile_keys + row;
+}
+// Its slot in the staged table, and the rows it reads (none if negative or zero).
+__host__ __device__ inline int rows_request_slot(int key, int paged_end, int lg) {
+  return (key < paged_end - 1 ? key : paged_end - 1) >> lg;
+}
+__host__ __device__ inline int rows_request_rows(int key, int paged_end) {
+  return paged_end - key < kRowsChunk ? paged_end - key : kRowsChunk;
+}
+
 // Slot of `key`'s block id in the staged table.
 __host__ __device__ inline int paged_stage_slot(int key, int kbeg, int lg) { return (key >> lg) - (kbeg >> lg); }
 
