@@ -667,6 +667,52 @@ def test_prefill_f32_few_keys(d, hq, lq, lk, causal):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n", [60, 150, 500])               # one, two, four key groups
+def test_prefill_f32_parts_of_weights_and_values(d, n):
+    """Equal values come out as they went in, whatever the weights: every part of a weight counts
+    against the row sum, which holds it whole, and every part of the value.  Six products,
+    their sum, the row sum's adds, the division and at most 2^-24 left out: 8 * 2^-24.  A part
+    product that is lost is 2^-17 of the value, over the root of the keys that matter."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    hq, hkv = 16, 8
+    q, k = randn(390, n, hq, d).cuda(), randn(391, n, hkv, d).cuda()
+    bits = np.random.default_rng(392).integers(0, 1 << 23, (hkv, d)) | 0x3f800000
+    bits[0], bits[1], bits[2] = 0x3f80ffff, 0x3f807fc0, 0x3f8080ff      # all low bits, the largest remainders
+    v = torch.from_numpy(bits.astype(np.int32)).view(torch.float32).expand(n, hkv, d).contiguous().cuda()
+    out = flash_prefill_attention(q[None], k[None], v[None])[0].double()
+    want = v[0].double().repeat_interleave(hq // hkv, 0)
+    assert ((out - want).abs() <= 8 * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_f32_parts_of_scores(d):
+    """Scores of one product each, x y / sqrt(d) = s against zero, with values 1 and -1: the output
+    is tanh(s / 2).  s errs by at most 2.5 * 2^-24 of it (one part product lost: 2^-17), an
+    exponential by 2^-22, and neither moves the output by more than half as much."""
+    from tinyvllm_amd.attention import flash_prefill_attention
+    n, m, hq, hkv = 64, 32, 32, 32
+    rng = np.random.default_rng(393)
+
+    def draw(*shape):
+        bits = rng.integers(0, 1 << 23, shape) | 0x3f800000
+        bits[::2] |= 0xffff
+        return torch.from_numpy(bits.astype(np.int32)).view(torch.float32)
+
+    x, y = draw(n, hq), draw(hkv)
+    dim = torch.from_numpy(rng.permutation(np.arange(hkv) * (d // hkv)))       # every 32-element step has some
+    q, k, v = torch.zeros(n, hq, d), torch.zeros(m, hkv, d), torch.zeros(m, hkv, d)
+    q[:, torch.arange(hq), dim] = x
+    k[0, torch.arange(hkv), dim] = y * d ** 0.5 / 2
+    k[2:, torch.arange(hkv), dim] = -1e4
+    v[0], v[1] = 1, -1
+    out = flash_prefill_attention(q.cuda()[None], k.cuda()[None], v.cuda()[None], False)[0].double().cpu()
+    s = x.double() * k[0, torch.arange(hkv), dim].double() * d ** -0.5
+    assert ((out - torch.tanh(s / 2)[:, :, None]).abs() <= (2.5 * s[:, :, None] + 8) * 2.0 ** -24 / 2).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
 def test_prefill_f32_positive_sums(d):
     """Equal weights over 32768 positive values: the sum of a key group's 512 (or 256) tiles
     walks by at most 2^-24 of it per tile, about sqrt(512) 2^-24 = 1.3e-6 in the end; the row sum
@@ -811,3 +857,22 @@ def test_prefill_paged_128_row_kernel_invalid_block_in_half_a_tile(dtype, out_dt
         out = flash_prefill_paged(q, kc, vc, table, start, out_dtype=out_dtype)[0]
         first = row // bs * bs // 64 * 64
         assert torch.isnan(out[first:]).all() and torch.equal(out[:first], good[:first])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("blocks", [2048, 2049])              # the longest table of the 128-row kernel, and one more
+def test_prefill_paged_128_row_kernel_longest_table(blocks):
+    from tinyvllm_amd.attention import flash_prefill_paged
+    hq, hkv, d, n, bs = 64, 8, 128, 1000, 4
+    start = blocks * bs - n
+    q, kc, vc = (randn(400 + i, *s, dtype=torch.bfloat16).cuda()
+                 for i, s in enumerate([(n, hq, d), (blocks + 1, bs, hkv, d), (blocks + 1, bs, hkv, d)]))
+    table = torch.from_numpy(np.random.default_rng(7).permutation(blocks + 1)[:blocks].astype(np.int32)).cuda()
+    out = flash_prefill_paged(q, kc, vc, table, start)[0].double()
+    k, v = (c[table.long()].reshape(-1, hkv, d).double() for c in (kc, vc))
+    rows = torch.tensor([0, 1, 31, 32, 127, 128, 500, n - 2, n - 1]).cuda()
+    for h in (0, 7, 8, 63):
+        s = q[rows, h].double() @ k[:, h // 8].T.contiguous() / d ** 0.5
+        s.masked_fill_(torch.arange(blocks * bs, device="cuda")[None] > rows[:, None] + start, -np.inf)
+        want = torch.softmax(s, -1) @ v[:, h // 8].contiguous()
+        assert (out[rows, h] - want).abs().max() < TOL[torch.bfloat16]

@@ -196,7 +196,95 @@ def test_linear_f32_many_rows(M, N, K, ks):
     check_products(torch.float32, M, N, K, ks)
 
 
-TILED_128, TILED_64 = 3, 4     # tv_linear_kernel: 128 x 128 and 64 x 128 tiles
+TILED_256, TILED_128, TILED_64 = 2, 3, 4     # tv_linear_kernel: 256 x 256, 128 x 128 and 64 x 128 tiles
+
+
+@pytest.mark.parametrize("dtype,M,N,K,ks,kernel", [
+    (dt, *c) for dt in (torch.float16, torch.bfloat16)
+    for c in ((129, 16388, 1056, 352, TILED_256), (129, 48004, 352, 352, TILED_256),
+              (65, 6148, 1056, 352, TILED_128), (65, 16388, 352, 352, TILED_128), (129, 48004, 480, 480, TILED_256),
+              (129, 2052, 1056, 352, TILED_64), (65, 8196, 352, 352, TILED_64))] + [
+    (torch.float32, *c) for c in ((65, 6148, 1056, 352, TILED_128), (65, 16388, 352, 352, TILED_128),
+                                  (65, 4100, 1056, 352, TILED_64), (65, 12292, 352, 352, TILED_64),
+                                  (129, 16388, 480, 480, TILED_64))])
+def test_linear_tiles(dtype, M, N, K, ks, kernel):
+    """Every tile shape past its ring (five and a half stages of 64 elements, eleven of 32), with
+    rows, features and a last stage that end inside it: partials of three splits, or logits,
+    keys and SwiGLU of one.  A rounding of the sum per MFMA and stage: (K / 8) 2^-24 of the sum
+    of magnitudes for exact 16-bit products, (K / 32 + 3) 2^-24 for fp32."""
+    from tinyvllm_amd._lib import dtype_code
+    code = dtype_code(dtype)
+    for epi in ((0,) if ks < K else (0, 1, 2)):
+        assert lib().tv_linear_kernel(M, N, K, ks, epi, code) == kernel
+    lda = K + 8
+    a = gen(52, M, lda, dtype=dtype)[:, :K]
+    w = gen(53, N, K, dtype=dtype, scale=0.05)
+    tol = (K / 32 + 3 if dtype == torch.float32 else K / 8) * 2.0 ** -24
+    A, W = a.double(), w.double()
+
+    def product(k=slice(None)):
+        return A[:, k] @ W[:, k].T.contiguous(), A[:, k].abs() @ W[:, k].abs().T.contiguous()
+
+    def run(out, ldo, epi, keys=None):
+        check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, lda, ldo, ks, epi, ptr(keys) if keys is not None else None,
+                              code, None), f"epilogue {epi}")
+        torch.cuda.synchronize()
+        return out.double()
+
+    part = run(torch.full((-(-K // ks), M, N), float("nan"), device="cuda"), 0, 0)
+    for s in range(part.shape[0]):
+        want, mag = product(slice(s * ks, (s + 1) * ks))
+        assert ((part[s] - want).abs() <= tol * mag).all(), s
+    if ks < K:
+        return
+    want, mag = product()
+    keys = torch.zeros((-(-N // 64), M), dtype=torch.int64, device="cuda")
+    logits = run(torch.full((M, N), float("nan"), device="cuda"), N, 2, keys)
+    assert ((logits - want).abs() <= tol * mag).all()
+    toks = torch.zeros(M, dtype=torch.int32, device="cuda")
+    check(lib().tv_argmax_advance(ptr(toks), None, None, None, 0, ptr(keys), keys.shape[0], M, None), "argmax")
+    torch.cuda.synchronize()
+    assert torch.equal(toks.long(), logits.argmax(1))
+    (g, u), (eg, eu) = [[x.view(M, N // 4, 2, 2)[:, :, i].reshape(M, -1) for i in (0, 1)] for x in (want, tol * mag)]
+    silu = g / (1 + torch.exp(-g))
+    bound = 1.1 * (u.abs() * eg + (g.abs() + eg) * eu) + (torch.finfo(dtype).eps / 2 * 1.01 + 2.0 ** -21) * (silu * u).abs()
+    sw = run(torch.full((M, N // 2), float("nan"), dtype=dtype, device="cuda"), N // 2, 1)
+    tiny = 0 if dtype != torch.float16 else 2.0 ** -24      # fp16 subnormals
+    assert ((sw - silu * u).abs() <= bound + tiny).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,ks", [(1, 4, 288, 288), (4, 1028, 864, 288), (3, 4100, 288, 288), (5, 516, 2080, 2080),
+                                      (8, 2052, 1632, 544), (16, 1028, 544, 544), (16, 8196, 2080, 1056)])
+def test_linear_few_rows_kernel(dtype, M, N, K, ks):
+    """The few-row kernel in its range, three types: waves without a stage, splits that are not
+    whole stages, rings that run across units, ragged N and K."""
+    from tinyvllm_amd._lib import dtype_code
+    for k, epi in ((ks, 0), (K, 1), (K, 2)):
+        assert lib().tv_linear_kernel(M, N, K, k, epi, dtype_code(dtype)) == 1
+    check_products(dtype, M, N, K, ks)
+
+
+@pytest.mark.parametrize("M,N,kernel", [(65, 16388, TILED_128), (65, 12292, TILED_64)])
+def test_linear_f32_tiles_non_finite(M, N, kernel):
+    """Infinities, NaN and values beyond the split's range give what fp32 products give."""
+    from tinyvllm_amd._lib import TV_F32
+    K = 160
+    assert lib().tv_linear_kernel(M, N, K, K, 2, TV_F32) == kernel
+    a, w = gen(54, M, K, dtype=torch.float32), gen(55, N, K, dtype=torch.float32, scale=0.05)
+    a[3, 5], a[20, 7], a[64, 1], a[33, 100] = float("inf"), float("nan"), 3.4e38, 2.0 ** 110
+    w[2, 9], w[131, 0], w[N - 1, K - 1] = float("-inf"), 3.4e38, float("nan")
+    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    check(lib().tv_linear(ptr(out), ptr(a), ptr(w), M, N, K, K, N, K, 2, None, TV_F32, None), "logits")
+    torch.cuda.synchronize()
+    want = a.double() @ w.double().T.contiguous()
+    want = torch.where(want.abs() > 3.4028235e38, want * float("inf"), want)
+    got = out.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    mag = torch.nan_to_num(a.double().abs(), nan=0, posinf=0) @ torch.nan_to_num(w.double().abs(), nan=0, posinf=0).T.contiguous()
+    assert ((got - want)[ok].abs() <= K * 2.0 ** -24 * mag[ok]).all()
 
 
 @pytest.mark.parametrize("M,N,kernel", [(65, 20484, TILED_128), (193, 6148, TILED_64)])
@@ -620,6 +708,35 @@ def test_f32_chunk_with_an_invalid_block(dim, heads, kv_heads, n, row):
     out = model.prefill_table(toks[start:], kv, table, start, attend_prefix=True)[0]
     assert torch.isnan(out[first:]).all()
     assert not first or max_err(out[:first].cpu().numpy(), good[:first].cpu().numpy()) < LOGIT_TOL["float32"]
+
+
+@pytest.mark.parametrize("dim,heads,kv_heads,start,n,block", [
+    (2048, 32, 4, 4, 60, 16),        # head_dim 64, one key group (up to 64 keys)
+    (1024, 16, 4, 100, 300, 4),      # four: 400 keys, 80 work-groups
+    (2048, 32, 4, 33, 130, 32),      # two
+    (7680, 60, 4, 4, 60, 16),        # head_dim 128, one
+    (4096, 32, 8, 33, 130, 4),       # two
+    (4096, 32, 8, 10, 1015, 16)])    # one: the grid fills every CU twice
+def test_f32_chunk_kernels(dim, heads, kv_heads, start, n, block):
+    """Each key grouping and head size of the paged fp32 kernel: a chunk after a prefix gives the
+    rows of one prefill of the whole prompt (one layer; weights that keep the logits' size).
+    Then an infinite and a NaN value in the prefix, in one KV head, reach the same rows."""
+    cfg = small_config(dim=dim, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, dtype="float32", max_seq_len=2048,
+                       hidden_dim=256)
+    from tinyvllm_amd.kv_cache import KVCache
+    from tinyvllm_amd.llama import Llama, random_weights
+    nb = -(-(start + n) // block) + 3
+    model = Llama(cfg, random_weights(cfg, seed=12, std=0.05 * (128 / dim) ** 0.5))
+    kv = KVCache(1, nb, block, kv_heads, dim // heads, cfg.dtype)
+    table = torch.randperm(nb, generator=torch.Generator().manual_seed(4)).int().cuda()
+    toks = np.random.default_rng(28).integers(0, cfg.vocab_size, start + n)
+    full = model.prefill_table(toks, kv, table, 0)[0]
+    chunk = model.prefill_table(toks[start:], kv, table, start, attend_prefix=True)[0]
+    assert max_err(chunk.cpu().numpy(), full[start:].cpu().numpy()) < LOGIT_TOL["float32"]
+    at = (int(table[0]), 1)                                  # position 1: every row of the chunk sees it
+    kv.v_cache[0][at][0, 3], kv.v_cache[0][at][kv_heads - 1, 5] = float("inf"), float("nan")
+    bad = model.prefill_table(toks[start:], kv, table, start, attend_prefix=True)[0]
+    assert not torch.isfinite(bad).any()
 
 
 def prefill_batch(model, kv, bm, ref, rk, rv, lens, rng, cfg):
