@@ -147,6 +147,18 @@ def test_kernel_of_a_many_row_product(dtype, M, N, K, splits, epilogue, tiled):
     assert kernel >= 2 if tiled else kernel == 0
 
 
+def test_a_planned_split_takes_the_kernel_it_was_planned_for():
+    """300 rows of 2048 x 2048 at fp32 are split eight ways for the tiled kernel (26 us); at that
+    split alone the estimates differ by 5%, and 64 x 64 tiles take 34."""
+    lib = _lib.load()
+    assert lib.tv_linear_kernel(300, 2048, 2048, 256, 0, _lib.TV_F32) >= 2
+    for M, N, K in ((1000, 2560, 2048), (300, 2048, 5632), (16, 2048, 2048), (65, 2048, 2048), (16, 4096, 1024)):
+        ks = lib.tv_linear_k_split(M, N, K)
+        want = {(16, 4096, 1024): 0}.get((M, N, K), 1 if M <= 16 else 2)
+        kernel = lib.tv_linear_kernel(M, N, K, ks, 0, _lib.TV_F16)
+        assert kernel >= 2 if want == 2 else kernel == want
+
+
 @pytest.mark.parametrize("dtype,M,N,K,epilogue,few", [
     # measured faster on 64 x 64 tiles: one or two chunks of K under many features
     ("F16", 4, 32768, 256, 1, False), ("F16", 16, 32768, 512, 1, False), ("BF16", 4, 8192, 256, 1, False),

@@ -517,20 +517,25 @@ static bool few_is_faster(int M, int N, int K, int k_split, int dtype, int epi) 
   return few_us(M, N, K, k_split, dtype) < skinny_us(M, N, K, k_split, dtype, false);
 }
 
-int linear_k_split(int M, int N, int K, int dtype) {
-  const int skinny = skinny_k_split(M, N, K);
-  double s = skinny_us(M, N, K, skinny, dtype, false);
+// Split of K and kernel of a product whose consumer sums the partials.
+struct SplitPlan {
+  int k_split;
+  LinearKernel kernel;
+};
+static SplitPlan split_plan(int M, int N, int K, int dtype) {
+  const SplitPlan skinny{skinny_k_split(M, N, K), kLinearSkinny};
+  if (M > kFewRows && M <= kLinBM) return skinny;
+  const double s = skinny_us(M, N, K, skinny.k_split, dtype, false) + partials_us(M, N, (K + skinny.k_split - 1) / skinny.k_split);
   if (M <= kFewRows) {
-    const int few = few_k_split(N, K, dtype == kF32 ? 4 : 2);
-    s += partials_us(M, N, (K + skinny - 1) / skinny);
-    return s <= few_us(M, N, K, few, dtype) ? skinny : few;
+    const SplitPlan few{few_k_split(N, K, dtype == kF32 ? 4 : 2), kLinearFew};
+    return s <= few_us(M, N, K, few.k_split, dtype) ? skinny : few;
   }
-  if (M <= kLinBM) return skinny;
-  const int tiled = dtype == kF32 ? tile_linear_f32_k_split(M, N, K) : tile_linear_k_split(M, N, K);
-  s += partials_us(M, N, (K + skinny - 1) / skinny);
-  const double t = tiled_us(M, N, K, tiled, dtype) + partials_us(M, N, (K + tiled - 1) / tiled);
+  const SplitPlan tiled{dtype == kF32 ? tile_linear_f32_k_split(M, N, K) : tile_linear_k_split(M, N, K), kLinearTiled};
+  const double t = tiled_us(M, N, K, tiled.k_split, dtype) + partials_us(M, N, (K + tiled.k_split - 1) / tiled.k_split);
   return s < t ? skinny : tiled;
 }
+
+int linear_k_split(int M, int N, int K, int dtype) { return split_plan(M, N, K, dtype).k_split; }
 
 // 32-bit offsets: in the 16 rows that few_linear_kernel addresses, and in the 16
 // rows of W and 64 of A (those past M too, which a wrapped offset would bring back
@@ -548,15 +553,18 @@ bool linear_supported(int M, int K, long long lda, int dtype) {
 }
 
 LinearKernel linear_kernel_of(const LinearParams& p, int epi, int dtype) {
-  if (p.M <= kFewRows) {
-    if (!few_supported(p.M, p.K, p.lda, dtype)) return kLinearSkinny;
-    return !skinny_supported(p.K, p.lda, dtype) || few_is_faster(p.M, p.N, p.K, p.k_split, dtype, epi) ? kLinearFew
-                                                                                                      : kLinearSkinny;
+  const bool few = few_supported(p.M, p.K, p.lda, dtype);
+  if (few && !skinny_supported(p.K, p.lda, dtype)) return kLinearFew;
+  const bool tiled = p.M > kLinBM && (dtype == kF32 ? tile_linear_f32_supported(p) : tile_linear_supported(p));
+  if (!few && !tiled) return kLinearSkinny;
+  if (epi == kEpiPartial) {   // the kernel that a planned split was made for; other splits are the caller's
+    const SplitPlan plan = split_plan(p.M, p.N, p.K, dtype);
+    if (plan.k_split == p.k_split) return plan.kernel;
   }
-  if (p.M > kLinBM && (dtype == kF32 ? tile_linear_f32_supported(p) : tile_linear_supported(p)) &&
-      tiled_us(p.M, p.N, p.K, p.k_split, dtype) <= skinny_us(p.M, p.N, p.K, p.k_split, dtype, epi == kEpiLogits))
-    return kLinearTiled;
-  return kLinearSkinny;
+  if (few) return few_is_faster(p.M, p.N, p.K, p.k_split, dtype, epi) ? kLinearFew : kLinearSkinny;
+  return tiled_us(p.M, p.N, p.K, p.k_split, dtype) <= skinny_us(p.M, p.N, p.K, p.k_split, dtype, epi == kEpiLogits)
+             ? kLinearTiled
+             : kLinearSkinny;
 }
 
 void launch_linear(const LinearParams& p, int epi, int dtype, hipStream_t s) {
