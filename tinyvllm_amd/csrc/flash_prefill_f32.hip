@@ -387,12 +387,14 @@ void launch_prefill_f32(const PrefillParams& p_in, hipStream_t s) {
   // Key groups shorten the chain of the longest row (about 1 us per 32 keys):
   // two beyond 64 keys (MI355X, Hq 32 / Hkv 4, head_dim 64, one / two: L 64 5.9 /
   // 6.1 us, L 300 17.9 / 13.8, L 1024 51.5 / 37.9, L 1500 77 / 72; head_dim 128,
-  // Hkv 8: L 512 40.2 / 31.9), but not at head_dim 128 where the grid fills every
-  // CU twice (L 1024 77 / 79, L 1500 145 / 153); four at head_dim 64 where it leaves
-  // CUs with one work-group (L 512 20.2 with two, 18.6; L 300 13.8, 13.7).
+  // Hkv 8: L 512 40.2 / 31.9), but not at head_dim 128 with two to three
+  // work-groups per CU, which one-group ones run at once (Hq 32, L 1300 106 / 124, L
+  // 1500 148 / 153; Hq 16, L 2500 195 / 207; beyond, Hq 32, L 1700 190 / 180); four
+  // at head_dim 64 where the grid leaves CUs with one work-group (L 512 20.2 with
+  // two, 18.6; L 300 13.8, 13.7).
   const long long wgs = (long long)p.num_heads * ((p.q_len + kBM - 1) / kBM);
   int ks = 2;
-  if (p.kv_len <= 64 || (p.head_dim == 128 && wgs >= 512)) ks = 1;
+  if (p.kv_len <= 64 || (p.head_dim == 128 && wgs > 512 && wgs <= 768)) ks = 1;
   else if (wgs <= 256 && p.kv_len >= 384) ks = 4;   // (head_dim 128: two)
   if (p.kv_table) launch_f32<true>(p, ks, s);
   else launch_f32<false>(p, ks, s);
