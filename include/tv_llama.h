@@ -54,7 +54,9 @@ int tv_linear_kernel(int M, int N, int K, int k_split, int epilogue, int dtype);
 /*
  * Y = A W^T, A [M, K] (row stride lda elements), W [N, K] dense, both of dtype.
  * Replaces tinygrad Linear(bias=False) calls (llama.py:150-153, 214-216, 254).
- * Requires K % 32 == 0, N % 4 == 0, k_split % 32 == 0, 16-byte aligned A/W rows.
+ * Requires K % 32 == 0, N % 4 == 0, k_split % 32 == 0, 16-byte aligned A/W rows;
+ * rows of at most 2^28 bytes in W and 2^26 in A (lda; 2^27 for at most 16 rows, any
+ * for one), TV_EUNSUPPORTED beyond.
  *  TV_EPI_PARTIAL: out float [ceil(K/k_split), M, N].
  *  TV_EPI_SWIGLU:  W rows 4j, 4j+1 are w1 rows 2j, 2j+1 and rows 4j+2, 4j+3 the
  *                  w3 rows 2j, 2j+1; out T [M, N/2] at row stride ldo

@@ -165,15 +165,16 @@ def check_products(dtype, M, N, K, ks):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (128, 128, 64, 64), (129, 132, 96, 96),      # 64 x 128 tiles
+@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (128, 128, 64, 64), (129, 132, 96, 96),
                                       (191, 260, 1056, 352), (320, 256, 2048, 512),
                                       (129, 16400, 160, 160),
-                                      (200, 32000, 128, 64), (257, 32772, 32, 32),                  # 128 x 128
-                                      (300, 32000, 96, 96), (513, 16392, 160, 160)])                # 256 x 256
+                                      (200, 32000, 128, 64), (257, 32772, 32, 32),
+                                      (300, 32000, 96, 96), (513, 16392, 160, 160)])
 def test_linear_many_rows(dtype, M, N, K, ks):
-    """More than 64 rows: each tile shape at its edges (rows, features and K past the last
-    tile, short last stages, splits that are not whole stages), A rows at a stride, the
-    three epilogues on the same products.  fp32 sums of exact products: the error of a sum
+    """More than 64 rows: sizes around the edges of every tile shape (rows, features and K past
+    the last tile, short last stages, splits that are not whole stages), on whichever kernel the
+    launcher takes (test_linear_tiles names them), A rows at a stride, the three epilogues on
+    the same products.  fp32 sums of exact products: the error of a sum
     of K terms is below K * 2^-24 of the sum of magnitudes, at most 2e-5 of it here."""
     check_products(dtype, M, N, K, ks)
 
@@ -188,11 +189,11 @@ def test_linear_few_rows(dtype, M, N, K, ks):
     check_products(dtype, M, N, K, ks)
 
 
-@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (64 + 33, 260, 96, 64), (129, 132, 1056, 352),   # 64 x 128 tiles
-                                      (321, 8260, 64, 64),                                            # several per CU
-                                      (300, 32000, 96, 96), (513, 16396, 32, 32)])                    # 128 x 128
+@pytest.mark.parametrize("M,N,K,ks", [(65, 4, 32, 32), (64 + 33, 260, 96, 64), (129, 132, 1056, 352),
+                                      (321, 8260, 64, 64), (300, 32000, 96, 96), (513, 16396, 32, 32)])
 def test_linear_f32_many_rows(M, N, K, ks):
-    """fp32 products from split operands: tile edges, one and many stages, the three epilogues."""
+    """fp32 products of many rows: sizes around tile edges, one and many stages, the three
+    epilogues, on whichever kernel the launcher takes."""
     check_products(torch.float32, M, N, K, ks)
 
 
@@ -716,7 +717,7 @@ def test_f32_chunk_with_an_invalid_block(dim, heads, kv_heads, n, row):
     (2048, 32, 4, 33, 130, 32),      # two
     (7680, 60, 4, 4, 60, 16),        # head_dim 128, one
     (4096, 32, 8, 33, 130, 4),       # two
-    (4096, 32, 8, 10, 1015, 16)])    # one: the grid fills every CU twice
+    (4096, 32, 8, 10, 1030, 16)])    # one: more than two work-groups per CU
 def test_f32_chunk_kernels(dim, heads, kv_heads, start, n, block):
     """Each key grouping and head size of the paged fp32 kernel: a chunk after a prefix gives the
     rows of one prefill of the whole prompt (one layer; weights that keep the logits' size).

@@ -106,7 +106,12 @@ def dtype_code(dt):
 
 def stream_ptr(device):
     """Handle of the current stream of a device (read without building a Stream
-    object, which took 2.0 of a decode call's 14.7 us on the host; this takes 0.2)."""
+    object, which took 2.0 of a decode call's 14.7 us on the host; this takes 0.2).
+
+    ``_cuda_getCurrentRawStream`` is private to torch (torch's own generated code
+    calls it); the public form of the same is
+    ``torch.cuda.current_stream(device).cuda_stream``.  It does not initialise the
+    device, which the tensors of every call have done."""
     import torch
     index = device.index if device.index is not None else torch.cuda.current_device()
     return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))

@@ -660,7 +660,7 @@ bool prefill_uses_mfma(const PrefillParams& p, int dtype) {
 // flash_prefill_rows.hip) for long head_dim-128 prompts, where they measured
 // faster (MI355X, Hq 32 / Hkv 8: L 2048 54-56 against 64-68 us, L 4096
 // 174 against 207-210); below 2048 rows, or at head_dim 64, this file's 64-row
-// kernel wins.
+// kernel wins.  (Chunks over a block table: use_rows_kernel_paged.)
 constexpr int kRowsMinLen = 2048;
 
 bool use_rows_kernel(int head_dim, long long max_q_len) { return head_dim == 128 && max_q_len >= kRowsMinLen; }
@@ -774,9 +774,9 @@ bool use_rows_kernel_paged(const PrefillParams& p) {
 }
 
 // One prompt whose keys and values are read through a block table
-// (kv_table set) with query rows at positions q_pos_offset ..: the 64-row
-// kernel with its loads going through the table.  Returns 1 when the shape has
-// no such kernel (fp32, head_dim other than 64 / 128, a block size that is
+// (kv_table set) with query rows at positions q_pos_offset ..: the 128-row or
+// the 64-row kernel with its loads going through the table.  Returns 1 when the
+// shape has no such kernel (fp32, head_dim other than 64 / 128, a block size that is
 // not a power of two, or more than kPagedTableMax blocks).
 int launch_flash_prefill_paged(const PrefillParams& p_in, int dtype, hipStream_t stream) {
   PrefillParams pp = p_in;

@@ -6,7 +6,9 @@
 // i when j > i with `causal` (top-left aligned), query head h on KV head
 // h / (Hq/Hkv), fp16 / bf16 inputs, fp32 accumulation.  Launched for head_dim
 // 128 (the kernel body is written for any head_dim whose tile fills the DMA
-// shape; at 64 the 64-row kernel was faster at every length measured).
+// shape; at 64 the 64-row kernel was faster at every length measured): prompts of
+// 2048 rows and more, and chunks over a block table whose grid gives every CU two
+// work-groups.
 //
 // Why a second kernel.  In the 64-row kernel every wave owns 16 query rows, so
 // each K / V byte read from LDS feeds 16 rows of MFMA work: at full matrix
@@ -48,8 +50,8 @@
 // causal): L 2048 54-56 us (51 us replayed in a graph) against 64-68 for the
 // 64-row kernel, L 4096 174 against 207-210; at L <= 1024 and at head_dim 64
 // the 64-row kernel is faster (L 512 / 1024 at head_dim 64: 7.6 / 13.0 us
-// against 12.1 / 20.7), so the launcher uses this one only for long
-// head_dim-128 prompts.  A tile step of the longest work-group takes ~2000
+// against 12.1 / 20.7), so among contiguous prompts the launcher uses this one
+// only for long head_dim-128 ones.  A tile step of the longest work-group takes ~2000
 // cycles against 512 of MFMA work (clock stamps): the LDS-DMA issue, LDS read
 // issue, score wait and softmax are serial within a wave, and with 2 waves per
 // SIMD (236 VGPRs fp16, 230 bf16) little of it overlaps.  Splitting a work-group's key tiles
